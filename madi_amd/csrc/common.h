@@ -23,6 +23,9 @@ int cu_count();
 // not freed, because graphs captured earlier still name it); all of them are
 // freed by madi_cleanup.
 int workspace(size_t partial_bytes, size_t counters, float **partials, uint32_t **cnt);
+// The same for a caller that has another way: false, with no error recorded,
+// where the workspace cannot grow (a graph capture, no memory).
+bool workspace_try(size_t partial_bytes, float **partials, uint32_t **cnt);
 // Releases the fp16 GEMM's rocBLAS handle (madi_cleanup).
 void f16gemm_cleanup();
 // The MFMA GEMM with f32 activations (rounded to f16) and an f32 result, for

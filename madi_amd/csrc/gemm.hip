@@ -73,6 +73,7 @@
 // overlap the conversion of the next), transposed so every global store
 // writes whole row segments of the tile (256 or 512 bytes, 16 per lane).
 #include "common.h"
+#include "gemm256.h"
 #include "vmem.h"
 
 using namespace madi;
@@ -1804,6 +1805,19 @@ bool use_tail(uint32_t splits, uint32_t chunks) {
 // Where a launch keeps its split-K partials and counters.
 enum Scratch { kWorkspace = 0, kStatic = 1 };
 
+// Scratch for a weight dequantised by the call (gemm256.hip), from where the
+// call's split-K partials would come; nullptr if there is not enough.
+void *weight_scratch(size_t bytes, Scratch where) {
+  if (where == kStatic) {
+    uint8_t *base = nullptr;
+    if (resolve_scratch(&base) != MADI_OK) return nullptr;
+    return base + kScratchCounters * 4;
+  }
+  float *ws = nullptr;
+  uint32_t *cnt = nullptr;
+  return workspace_try(bytes, &ws, &cnt) ? ws : nullptr;
+}
+
 template <int MT, int EPI, bool F32 = false, int PW = 2>
 int launch_gemm(const void *A, const uint8_t *qs, const f16 *sc, void *C, const float *bias,
                 uint32_t M, uint32_t N, uint32_t K, Scratch where, const OutSeg &seg = OutSeg{}) {
@@ -1949,6 +1963,13 @@ int q8_gemm(const char *what, const void *a, const void *qs, const void *scales,
   if (tile_count(m, n, 3) <= cus)
     return dispatch_epi<3>(epilogue, A, Q, S, C, bias, m, n, k, where, seg);
   if (seg.n) return kSegUnsupported;
+  // many rows: 256 x 256 tiles on the weight dequantised once into scratch,
+  // where the fixed array holds it too (so that both entry points take the
+  // same kernel).  A workspace that would have to grow during a graph capture
+  // leaves the call to the kernels below.
+  if (gemm256_suits(m, n, k, kScratchBytes - kScratchCounters * 4))
+    if (void *w16 = weight_scratch(gemm256_bytes(n, k), where))
+      return gemm256(A, Q, S, C, bias, m, n, k, epilogue, w16);
   // at least two rounds of 128-row tiles: the persistent tile loop
   if (persist_ok(m, n, k)) {
     switch (epilogue) {

@@ -1,0 +1,113 @@
+"""The 256 x 256 tiles of the many-row Q8 GEMM (madi_amd/csrc/gemm256.hip)
+through the C ABI, against the oracle and element-wise against the exact
+product (fp32 accumulation plus one f16 rounding)."""
+import numpy as np
+import pytest
+
+import oracle as O
+from madi_amd import _lib, synth
+from test_gpu_q8 import TOL, dev, dev_f16, host_f16, normwise, say, tight_epi_ok, tight_ok
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+EPI = [O.EPI_NONE, O.EPI_BIAS, O.EPI_BIAS_GELU]
+
+
+@pytest.fixture(scope="module")
+def q():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import madi_amd.q8 as q8
+    q8.init()
+    return q8
+
+
+def check(c, a, qs, sc, bias, epi, rows):
+    b = None if epi == O.EPI_NONE else bias
+    ref = O.q8_gemm_rows(a, qs, sc, rows=rows, bias=b, epilogue=epi, threads=16)
+    assert normwise(c[rows], ref) <= TOL
+    if epi == O.EPI_NONE:
+        assert tight_ok(c[rows], a[rows], qs, sc)
+    else:
+        assert tight_epi_ok(c[rows], a[rows], qs, sc, bias, epi == O.EPI_BIAS_GELU)
+    assert np.all(np.isfinite(c))
+
+
+# One tile per CU (streams of one, two, three and four chunks; row tails of 65
+# rows and more), two rounds with an uneven second one, three tiles per
+# workgroup with a row tail of one.
+@pytest.mark.parametrize("m,n,k,epi", [
+    (65, 65536, 64, O.EPI_NONE), (256, 59136, 128, O.EPI_BIAS), (500, 29696, 192, O.EPI_BIAS_GELU),
+    (600, 20480, 256, O.EPI_NONE), (1900, 15872, 192, O.EPI_BIAS_GELU), (2305, 19456, 64, O.EPI_BIAS),
+    (6000, 5120, 1280, O.EPI_BIAS_GELU),
+])
+def test_tiles_against_oracle(q, m, n, k, epi):
+    say(f"gemm256 m={m} n={n} k={k} epi={epi}")
+    a, qs, sc = synth.gemm_case(m + k, m, n, k)
+    bias = np.random.default_rng(m).standard_normal(n).astype(np.float32)
+    w = q.upload_q8(qs, sc)
+    big = torch.full((m + 8, n), 0x7E00, dtype=torch.int16, device="cuda")  # rows past M stay
+    a_d, b_d = dev_f16(a), dev(bias)
+    call = lambda name: _lib.call(name, a_d.data_ptr(), w.qs, w.scales, big.data_ptr(),
+                                  None if epi == O.EPI_NONE else b_d.data_ptr(), m, n, k, epi)
+    call("madi_q8_gemm")
+    q.sync()
+    out = big.cpu().numpy()
+    assert np.all(out[m:] == 0x7E00)
+    edges = np.arange(128, m, 128)
+    rows = np.unique(np.r_[0, 15, 16, 63, 64, m // 2, m - 2, m - 1, edges[:8] - 1, edges[:8]])
+    check(host_f16(big)[:m], a, qs, sc, bias, epi, rows)
+    # again, and through the fixed scratch: the same bits
+    for name in ("madi_q8_gemm", "madi_q8_gemm_noalloc"):
+        big.fill_(0x7E00)
+        call(name)
+        q.sync()
+        assert np.array_equal(big.cpu().numpy(), out), name
+
+
+def test_capture_before_and_after_the_scratch_grows(q):
+    """With the workspace at its initial 4 MiB the 13 MB weight of 6000 x 1280
+    -> 5120 does not fit and may not be allocated for during a capture: the
+    captured call takes the fused kernels.  After an eager call has grown the
+    workspace a capture takes the 256 x 256 tiles.  Every replay of both, with
+    eager calls between, is within the bounds and repeats its own bits."""
+    m, n, k = 6000, 5120, 1280
+    say(f"gemm256 capture m={m} n={n} k={k}")
+    _lib.lib().madi_cleanup()
+    q.init()
+    a, qs, sc = synth.gemm_case(5, m, n, k)
+    bias = np.random.default_rng(6).standard_normal(n).astype(np.float32)
+    w = q.upload_q8(qs, sc)
+    a_d, b_d = dev_f16(a), dev(bias)
+    rows = np.unique(np.r_[0, 127, 128, 255, 256, 3000, m - 1])
+    graphs = []
+    for _ in range(2):
+        c = torch.empty((m, n), dtype=torch.int16, device="cuda")
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            with torch.cuda.graph(g, stream=side):
+                q.init(side)
+                q.kGemmQ8Bias(a_d, w, c, b_d, m, n, k, gelu=True)
+        q.init()
+        graphs.append((g, c))
+        eager = torch.empty((m, n), dtype=torch.int16, device="cuda")
+        q.kGemmQ8Bias(a_d, w, eager, b_d, m, n, k, gelu=True)
+        q.sync()
+    first = [None, None]
+    for rep in range(3):
+        for i, (g, c) in enumerate(graphs):
+            c.fill_(-1)
+            g.replay()
+            torch.cuda.synchronize()
+            got = host_f16(c)
+            if rep == 0:
+                first[i] = got.copy()
+                check(got, a, qs, sc, bias, O.EPI_BIAS_GELU, rows)
+            assert np.array_equal(got.view(np.uint16), first[i].view(np.uint16)), (rep, i)
+            q.kGemmQ8Bias(a_d, w, eager, b_d, m, n, k, gelu=True)
+            q.sync()
+    assert np.array_equal(host_f16(eager).view(np.uint16), first[1].view(np.uint16))
