@@ -1,46 +1,52 @@
-// gemv.hip -- decoder Q8 GEMV family (M = 1), HBM-bound.
+// gemv.hip -- decoder Q8 GEMV family (M = 1).
 //
 // Replaces gemv_q8 / _bias / _bias_gelu / _bias_res / _qkv and logit_gemv_q8
 // (engine/metal/kernels/graph_helpers.metal:320-558).  The reference runs one
-// 32-lane simdgroup per output row reading char4 + float4; here a workgroup
-// owns one 32-row panel of the panel layout and its waves split K: four for
-// the vocab matrix, sixteen for the decoder's 40 - 160-panel matrices (so a
-// K = 1280 range is one round of loads).  Every wave64 load instruction moves
-// one contiguous KiB (16 bytes per lane, lane (h, r) receiving 16 weights of
-// row r in quantisation block h), issued as a buffer load with the
-// panel/chunk offset in an SGPR.  Each wave streams its K range through a
-// two-chunk window (use chunk c, refill with chunk c+2).  The four-wave
-// instances keep to 62 - 71 VGPRs (seven waves per SIMD allow 72), so every workgroup
-// of the 51866-row vocab matrix (1621 panels, seven per CU) is resident from
-// the start; the sixteen-wave ones (four waves per SIMD) take up to 94.
+// 32-lane simdgroup per output row reading char4 + float4; here two kernels
+// share the arithmetic and the epilogues.
 //
-// The activation vector is loaded next to the first weight window (before
-// it for the narrow matrices, after it for the vocab), staged once per
+// q8_gemv_kernel, the vocab matrix and other wide ones (HBM-bound): a
+// workgroup of four waves owns one 32-row panel of the panel layout and its
+// waves split K.  Every wave64 load instruction moves one contiguous KiB (16
+// bytes per lane, lane (h, r) receiving 16 weights of row r in quantisation
+// block h), issued as a buffer load with the panel/chunk offset in an SGPR.
+// Each wave streams its K range through a two-chunk window (use chunk c,
+// refill with chunk c+2).  62 - 71 VGPRs (seven waves per SIMD allow 72), so
+// every workgroup of the 51866-row vocab matrix (1621 panels, seven per CU)
+// is resident from the start.
+//
+// q8_gemv_rows_kernel, the decoder's projections (latency-bound): a workgroup
+// owns 8 or 16 rows and all of K (below).
+//
+// The activation vector is loaded next to the first weights (after them for
+// the wide matrices, before them for the narrow ones), staged once per
 // workgroup in LDS and read back as broadcast 128-bit LDS loads, ahead of
-// the weights they meet (the narrow matrices' first window while its weights
-// are in flight; the vocab's fp32 vector one 16-value unit ahead).  v_perm_b32
-// turns two stored bytes u = q + 128 into the fp16 pair 1024 + u and one
-// packed subtract of 1152 leaves the exact fp16 pair (q0, q1); fp16
-// activations accumulate x * q with v_dot2_f32_f16 (exact products, fp32
-// sums), fp32 activations with FMA.  Per quantisation block the lane
-// multiplies its partial by the block's scale, the (partial * scale)
-// structure of the reference's kernels; the two K-halves meet by a cross-lane
-// shuffle and the four waves through LDS.  (Accumulating x * (1024 + u) and
-// subtracting 1152 * sum(x) per block saves the subtract but cancels two
-// large sums: an all-zero block, whose scale is 1.0, then leaks ~1e-2 of
-// rounding noise into its row.)
+// the weights they meet.  v_perm_b32 turns two stored bytes u = q + 128 into
+// the fp16 pair 1024 + u and one packed subtract of 1152 leaves the exact
+// fp16 pair (q0, q1); fp16 activations accumulate x * q with v_dot2_f32_f16
+// (exact products, fp32 sums), fp32 activations with FMA.  Each lane's
+// partial over (its half of) a quantisation block is multiplied by the
+// block's scale, the (partial * scale) structure of the reference's kernels;
+// lanes meet by cross-lane operations and waves through LDS.  (Accumulating
+// x * (1024 + u) and subtracting 1152 * sum(x) per block saves the subtract
+// but cancels two large sums: an all-zero block, whose scale is 1.0, then
+// leaks ~1e-2 of rounding noise into its row.)
+//
+// Kernel arguments: pointers travel as integers and only what a kernel uses
+// is passed.  Host cost of a launch (one box, an empty kernel of 40 x 1024
+// threads, no argument 1.2 us): ten pointers 3.7 us, the same ten as 64-bit
+// integers 2.8 us (the runtime looks every pointer argument up), 64 bytes
+// 2.7, 128 bytes 3.4.  At 2.5 - 3.5 us a kernel the decoder's projections
+// were bound by that.
 #include "common.h"
 
 using namespace madi;
 
 namespace {
 
-// Waves per workgroup (K ranges per panel): four for wide matrices (the
-// vocab logits: 1621 panels, seven workgroups per CU); sixteen below
-// kWidePanels, where four waves would each walk five chunks of a K = 1280
-// row through the window (three rounds of memory latency) on fewer than
-// half the CUs.
-constexpr int kWaves = 4, kWavesNarrow = 16;
+// Waves per panel of the wide kernel (seven workgroups per CU), which takes
+// matrices of at least kWidePanels panels.
+constexpr int kWaves = 4;
 constexpr uint32_t kWidePanels = 256;
 // Chunks in flight per wave, a sliding window: two keeps ~26 MB of the vocab
 // matrix in flight across the GPU, enough to cover HBM latency, while the
@@ -64,17 +70,16 @@ struct GemvArgs {
   const float *qb, *vb;
   float *kc, *vc;
   const uint32_t *pos;
-  // split K over `splits` workgroups per panel: partial row sums in `ws`
-  // ([panel][split][32]), arrival counters in `cnt` ([panel], zero between uses)
-  uint32_t splits;
-  float *ws;
-  uint32_t *cnt;
 };
 
-// LDS bytes: x (K elements of XT), the KW waves' partials
-template <typename XT, int KW>
+typedef __attribute__((address_space(1))) float gfloat;
+typedef __attribute__((address_space(1))) uint32_t guint;
+inline uint64_t addr(const void *p) { return reinterpret_cast<uint64_t>(p); }
+
+// LDS bytes of the wide kernel: x (K elements of XT), the waves' partials
+template <typename XT>
 constexpr size_t lds_bytes(uint32_t k) {
-  return (size_t)k * sizeof(XT) + KW * 32 * 4;
+  return (size_t)k * sizeof(XT) + kWaves * 32 * 4;
 }
 
 // One chunk's loads for a lane: its two 16-byte units and its block's scale.
@@ -169,68 +174,90 @@ __device__ inline void accumulate(const ChunkW &b, uint32_t c, const XT *xs, uin
   accumulate_x(b, xs + c * kChunkK + h * 32, acc);
 }
 
+// The epilogue's operands of one output row, loaded behind the first weights
+// so their latency passes during the K loop, and its store.
+struct RowEpi {
+  float bias = 0.0f, res = 0.0f;
+  uint32_t pos = 0;
+};
+template <int MODE>
+__device__ inline RowEpi epi_load(bool mine, uint32_t row, uint32_t K, const gfloat *out,
+                                  const gfloat *bias, const gfloat *vb, const guint *pos) {
+  RowEpi e;
+  if (mine) {
+    if constexpr (MODE == kBias || MODE == kBiasGelu) {
+      e.bias = bias[row];
+    } else if constexpr (MODE == kBiasRes) {
+      e.bias = bias[row];
+      e.res = out[row];
+    } else if constexpr (MODE == kQkv) {  // bias: q's
+      if (row < K) e.bias = bias[row];
+      else if (row >= 2 * K) e.bias = vb[row - 2 * K];
+    }
+  }
+  if constexpr (MODE == kQkv) e.pos = pos[0];
+  return e;
+}
+template <int MODE>
+__device__ inline void epi_store(float v, const RowEpi &e, uint32_t row, uint32_t K, gfloat *out,
+                                 gfloat *kc, gfloat *vc) {
+  if constexpr (MODE == kPlain) {
+    out[row] = v;
+  } else if constexpr (MODE == kBias) {
+    out[row] = v + e.bias;
+  } else if constexpr (MODE == kBiasGelu) {
+    out[row] = gelu_erf(v + e.bias);
+  } else if constexpr (MODE == kBiasRes) {
+    out[row] = e.res + v + e.bias;
+  } else {  // kQkv: n = 3 D, K = D
+    if (row < K)
+      out[row] = v + e.bias;
+    else if (row < 2 * K)
+      kc[(size_t)e.pos * K + (row - K)] = v;
+    else
+      vc[(size_t)e.pos * K + (row - 2 * K)] = v + e.bias;
+  }
+}
+
 template <typename XT>
 constexpr bool kBlockF32 = sizeof(XT) == 4;
 
-// Narrow matrices: sixteen waves of one panel, four per SIMD, so up to 128
-// VGPRs each (the first window's activations are held in registers, below).
-template <int KW>
-constexpr int kWavesPerEu = KW == kWavesNarrow ? 4 : 7;
-
-template <typename XT, int MODE, int KW>
-//
-// Grid (x, y) = (panel, K split).  The arguments are scalars in the order the
-// kernel first needs them, so the leading ones arrive preloaded in SGPRs, and
-// the set-up has no integer division: split s covers chunks [s * cper +
-// min(s, crem), + cper + (s < crem)).
-__global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<KW>))) void q8_gemv_kernel(
-    const uint8_t *qs, const f16 *sc, const void *x, uint32_t n, uint32_t k, uint32_t cper,
-    uint32_t crem, float *out, const float *bias, float *wsp, uint32_t *cnt, const float *qb,
-    const float *vb, float *kc, float *vc, const uint32_t *pos) {
-  const GemvArgs a{out, x, qs, sc, bias, n, k, qb, vb, kc, vc, pos, gridDim.y, wsp, cnt};
+// Grid: one workgroup per panel.  bias is q's for the QKV mode.
+template <typename XT, int MODE>
+__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(7))) void q8_gemv_kernel(
+    uint64_t qs_, uint64_t sc_, uint64_t x_, uint32_t n, uint32_t K, uint64_t out_, uint64_t bias_,
+    uint64_t vb_, uint64_t kc_, uint64_t vc_, uint64_t pos_) {
+  constexpr int KW = kWaves;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  const uint32_t K = a.k;
   XT *xs = reinterpret_cast<XT *>(smem);                        // [K]
-  float *red = reinterpret_cast<float *>(smem + lds_bytes<XT, KW>(K) - KW * 32 * 4);  // [KW][32]
+  float *red = reinterpret_cast<float *>(smem + (size_t)K * sizeof(XT));  // [KW][32]
 
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t h = lane >> 5, r = lane & 31;
-  const uint32_t p = blockIdx.x, split = blockIdx.y;
-  const uint32_t R = panel_rows(a.n, p);
+  const uint32_t p = blockIdx.x;
+  const uint32_t R = panel_rows(n, p);
   const bool live = r < R;
-  // this workgroup's K chunks [cs, cs + nck), split KW ways over the waves
-  const uint32_t cs = split * cper + (split < crem ? split : crem);
-  const uint32_t nck = cper + (split < crem ? 1 : 0);
-  const uint32_t c0 = cs + (wave * nck) / KW, c1 = cs + ((wave + 1) * nck) / KW;
+  const uint32_t chunks = K / kChunkK;
+  const uint32_t c0 = (wave * chunks) / KW, c1 = ((wave + 1) * chunks) / KW;
 
-  // ---- x (16 bytes per thread and piece) and the first weight window.
-  // Narrow matrices (sixteen waves, one or two chunks each) load x first: its
-  // staging barrier, not the weights, is then the longer wait.  The vocab
-  // matrix (four waves, five chunks each) issues its first weight window
-  // first, so the HBM requests leave before the L2-resident vector's
-  // (alternating runs in one process: 12.16 -> 11.92 us with f16 x, 12.66 ->
-  // 12.35 us with f32 x; the narrow ones measured slower that way, a decoder
-  // token 126 -> 134 us).  Lanes past a partial panel's last row read row R-1
-  // (in bounds; their sums are never stored).
-  constexpr bool kWeightsFirst = KW == kWaves;
+  // ---- The first weight window, then x (16 bytes per thread and piece), so
+  // the HBM requests leave before the L2-resident vector's (alternating runs
+  // in one process: 12.16 -> 11.92 us with f16 x, 12.66 -> 12.35 us with f32
+  // x).  Lanes past a partial panel's last row read row R-1 (in bounds; their
+  // sums are never stored).
   const uint32_t pieces = K * sizeof(XT) / 16;
-  const rsrc_t xr = make_rsrc(a.x, K * sizeof(XT));
+  const rsrc_t xr = make_rsrc((const void *)x_, K * sizeof(XT));
   u32x4 xv0 = {}, xv1 = {};
   const uint32_t i0 = threadIdx.x, i1 = threadIdx.x + KW * 64;
-  if constexpr (!kWeightsFirst) {
-    if (i0 < pieces) xv0 = __builtin_amdgcn_raw_buffer_load_b128(xr, i0 * 16, 0, 0);
-    if (i1 < pieces) xv1 = __builtin_amdgcn_raw_buffer_load_b128(xr, i1 * 16, 0, 0);
-  }
-
-  const rsrc_t wq = make_rsrc(a.qs, a.n * K), ws = make_rsrc(a.sc, a.n * (K / 32) * 2);
+  const rsrc_t wq = make_rsrc((const void *)qs_, n * K), ws = make_rsrc((const void *)sc_, n * (K / 32) * 2);
   // chunks past the wave's range load through an empty resource: no memory
   // access, zeros returned, so their scale is 0 and they add exactly nothing.
   // Every window load is then unconditional, which keeps each window slot in
   // the same registers from trip to trip (a conditional load makes the
   // compiler copy the slot at the loop back edge, and a copy must first wait
   // for the load that was just issued, collapsing the window).
-  const rsrc_t wz = make_rsrc(a.qs, 0);
+  const rsrc_t wz = make_rsrc((const void *)qs_, 0);
   const uint32_t rr = live ? r : R - 1;
   const uint32_t w_voff = (h * R + rr) * 16, s_voff = (h * R + rr) * 2;
   // the first kWin chunks of this wave's range
@@ -240,29 +267,13 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(kWavesP
     const bool in = c0 + k < c1;
     load_chunk(win[k], in ? wq : wz, in ? ws : wz, K, c0 + k, p, R, w_voff, s_voff);
   }
-  if constexpr (kWeightsFirst) {
-    if (i0 < pieces) xv0 = __builtin_amdgcn_raw_buffer_load_b128(xr, i0 * 16, 0, 0);
-    if (i1 < pieces) xv1 = __builtin_amdgcn_raw_buffer_load_b128(xr, i1 * 16, 0, 0);
-  }
+  if (i0 < pieces) xv0 = __builtin_amdgcn_raw_buffer_load_b128(xr, i0 * 16, 0, 0);
+  if (i1 < pieces) xv1 = __builtin_amdgcn_raw_buffer_load_b128(xr, i1 * 16, 0, 0);
 
-  // The epilogue's operands (bias, residual, q/v bias, cache position) load
-  // now, behind the weights, so their latency passes during the K loop
-  // instead of after it.  Lanes 0..R-1 of wave 0 own the panel's rows.
+  // lanes 0..R-1 of wave 0 own the panel's rows
   const uint32_t erow = p * kPanelRows + threadIdx.x;
-  float e_bias = 0.0f, e_res = 0.0f;
-  uint32_t e_pos = 0;
-  if (threadIdx.x < R) {
-    if constexpr (MODE == kBias || MODE == kBiasGelu) {
-      e_bias = a.bias[erow];
-    } else if constexpr (MODE == kBiasRes) {
-      e_bias = a.bias[erow];
-      e_res = a.out[erow];
-    } else if constexpr (MODE == kQkv) {
-      if (erow < a.k) e_bias = a.qb[erow];
-      else if (erow >= 2 * a.k) e_bias = a.vb[erow - 2 * a.k];
-    }
-  }
-  if constexpr (MODE == kQkv) e_pos = a.pos[0];
+  const RowEpi epi = epi_load<MODE>(threadIdx.x < R, erow, K, (const gfloat *)out_, (const gfloat *)bias_,
+                                    (const gfloat *)vb_, (const guint *)pos_);
 
   // stage x
   for (uint32_t i = threadIdx.x; i < pieces; i += KW * 64) {
@@ -276,33 +287,7 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(kWavesP
   // registers with chunk c + kWin
   float acc = 0.0f;
   uint32_t cfirst = c0;
-  if constexpr (KW == kWavesNarrow) {
-    // Narrow matrices (one or two chunks per wave): the first window's
-    // activations are read from LDS now, while its weights are still in
-    // flight, instead of after they land, when all sixteen waves would queue
-    // at the LDS at once.
-    if (c0 < c1) {
-      XT xf[kWin][32];
-#pragma unroll
-      for (int k = 0; k < kWin; ++k) {
-        const uint32_t cc = c0 + k < c1 ? c0 + k : c1 - 1;
-#pragma unroll
-        for (int i = 0; i < 32; ++i) xf[k][i] = xs[cc * kChunkK + h * 32 + i];
-      }
-      // the reads stay ahead of the first wait for the weights
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int k = 0; k < kWin; ++k) {
-        accumulate_x<XT>(win[k], xf[k], acc);
-        const uint32_t cn = c0 + k + kWin;
-        const bool in = cn < c1;
-        load_chunk(win[k], in ? wq : wz, in ? ws : wz, K, cn, p, R, w_voff, s_voff);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      cfirst = c0 + kWin;
-    }
-  }
-  if constexpr (KW == kWaves && kBlockF32<XT>) {
+  if constexpr (kBlockF32<XT>) {
     // The vocab matrix with fp32 activations: each unit's activations are
     // read from LDS one unit ahead of their use (the next chunk's first unit
     // during this chunk's second), so the LDS latency passes under the
@@ -354,54 +339,239 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(kWavesP
   if (h == 0) red[wave * 32 + r] = acc;
   __syncthreads();
   const uint32_t t = threadIdx.x;
-  float v = 0.0f;
-  if (t < 32) {  // the waves' partials in wave order
-    v = red[t];
-#pragma unroll
-    for (int w = 1; w < KW; ++w) v += red[w * 32 + t];
-  }
-  if (a.splits > 1) {
-    // Split K: each workgroup writes its 32 partial row sums past its XCD's L2
-    // (device-scope stores) and counts itself in with a device-scope atomic
-    // (every party is a workgroup of this launch); the last to arrive adds the
-    // splits' partials in split order (the same order whoever arrives last)
-    // and stores the rows.
-    __shared__ uint32_t arrived;
-    float *mine = a.ws + ((size_t)p * a.splits + split) * 32;
-    if (t < 32) __hip_atomic_store(mine + t, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (t == 0)
-      arrived = __hip_atomic_fetch_add(&a.cnt[p], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (arrived != a.splits - 1) return;
-    if (t < 32) {
-      const float *all = a.ws + (size_t)p * a.splits * 32 + t;
-      v = 0.0f;
-      for (uint32_t s2 = 0; s2 < a.splits; ++s2)
-        v += __hip_atomic_load(all + s2 * 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (t == 0) __hip_atomic_store(&a.cnt[p], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
   if (t >= R) return;
-  const uint32_t nrow = erow;  // t == threadIdx.x
-  if constexpr (MODE == kPlain) {
-    a.out[nrow] = v;
-  } else if constexpr (MODE == kBias) {
-    a.out[nrow] = v + e_bias;
-  } else if constexpr (MODE == kBiasGelu) {
-    a.out[nrow] = gelu_erf(v + e_bias);
-  } else if constexpr (MODE == kBiasRes) {
-    a.out[nrow] = e_res + v + e_bias;
-  } else {  // kQkv: a.n = 3D, a.k = D
-    const uint32_t D = a.k, pos = e_pos;
-    if (nrow < D)
-      a.out[nrow] = v + e_bias;
-    else if (nrow < 2 * D)
-      a.kc[(size_t)pos * D + (nrow - D)] = v;
-    else
-      a.vc[(size_t)pos * D + (nrow - 2 * D)] = v + e_bias;
+  float v = red[t];  // the waves' partials in wave order
+#pragma unroll
+  for (int w = 1; w < KW; ++w) v += red[w * 32 + t];
+  epi_store<MODE>(v, epi, erow, K, (gfloat *)out_, (gfloat *)kc_, (gfloat *)vc_);
+}
+
+// ---- narrow matrices (fewer than kWidePanels panels: the decoder's
+// projections), one workgroup per 8 NR rows.
+//
+// These are 1.7 - 7 MB each, so a launch is latency and, per CU, arithmetic:
+// a workgroup per 32-row panel left a 1280-row projection on 40 of the 256
+// CUs with four waves per SIMD of dequantisation and FMAs, and a K of 5120
+// had to be split over workgroups that met through memory.  Here a wave's
+// load takes 8 rows x 2 chunks (eight whole 128-byte lines of the panel
+// layout: lane (u, row) gets unit u % 4 of chunk u / 4), so a workgroup can
+// own as few as 8 rows with all of K, and its waves meet in LDS only.
+constexpr int kRowWaves = 16;
+
+// One pair of chunks: NR row groups' units and scales.
+template <int NR>
+struct PairW {
+  u32x4 w[NR];
+  uint32_t s[NR];
+};
+
+__device__ inline float xunit_dot(const u32x4 &w, const f32x4 (&x)[4]) {
+  const uint32_t wd[4] = {w.x, w.y, w.z, w.w};
+  float part = 0.0f;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const f16x2 q01 = q_pair(wd[d], kSelLo), q23 = q_pair(wd[d], kSelHi);
+    part = __builtin_fmaf(x[d].x, (float)q01.x, part);
+    part = __builtin_fmaf(x[d].y, (float)q01.y, part);
+    part = __builtin_fmaf(x[d].z, (float)q23.x, part);
+    part = __builtin_fmaf(x[d].w, (float)q23.y, part);
   }
+  return part;
+}
+__device__ inline float xunit_dot(const u32x4 &w, const f16x8 (&x)[2]) {
+  const uint32_t wd[4] = {w.x, w.y, w.z, w.w};
+  float part = 0.0f;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const f16x8 &xv = x[d / 2];
+    const int e = (d & 1) * 4;
+    part = __builtin_amdgcn_fdot2(q_pair(wd[d], kSelLo), (f16x2){xv[e], xv[e + 1]}, part, false);
+    part = __builtin_amdgcn_fdot2(q_pair(wd[d], kSelHi), (f16x2){xv[e + 2], xv[e + 3]}, part, false);
+  }
+  return part;
+}
+template <typename XT>
+struct XUnitOf;
+template <>
+struct XUnitOf<float> {
+  f32x4 v[4];
+};
+template <>
+struct XUnitOf<f16> {
+  f16x8 v[2];
+};
+__device__ inline void read_x(XUnitOf<float> &u, const float *x) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) u.v[i] = *reinterpret_cast<const f32x4 *>(x + 4 * i);
+}
+__device__ inline void read_x(XUnitOf<f16> &u, const f16 *x) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) u.v[i] = *reinterpret_cast<const f16x8 *>(x + 8 * i);
+}
+
+// the sum over the lanes with the same lane % 8
+__device__ inline float sum_units(float v) {
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xf,
+                                                             0xf, true));  // row_ror:8
+  const uint32_t a = __builtin_bit_cast(uint32_t, v);
+  const auto s16 = __builtin_amdgcn_permlane16_swap(a, a, false, false);
+  v = __builtin_bit_cast(float, (uint32_t)s16[0]) + __builtin_bit_cast(float, (uint32_t)s16[1]);
+  const uint32_t b = __builtin_bit_cast(uint32_t, v);
+  const auto s32 = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  return __builtin_bit_cast(float, (uint32_t)s32[0]) + __builtin_bit_cast(float, (uint32_t)s32[1]);
+}
+
+constexpr uint32_t kNowhere = 0x80000000u;  // past every buffer (operands stay below 2 GiB)
+
+template <typename XT, int MODE, int NR, int WIN, bool ONE>
+__device__ inline void gemv_rows(uint64_t x_, uint64_t qs_, uint32_t n, uint32_t K, uint64_t sc_,
+                                 uint64_t out_, uint64_t bias_, uint64_t vb_, uint64_t kc_, uint64_t vc_,
+                                 uint64_t pos_) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  XT *xs = reinterpret_cast<XT *>(smem);                                  // [K]
+  float *red = reinterpret_cast<float *>(smem + (size_t)K * sizeof(XT));  // [waves][8 NR]
+  constexpr uint32_t kRows = 8 * NR;
+  const uint32_t chunks = K / kChunkK, pairs = (chunks + 1) / 2;
+  const uint32_t waves = ONE ? (pairs + WIN - 1) / WIN : kRowWaves, threads = waves * 64;
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t row0 = blockIdx.x * kRows;  // of 32-row panel p
+  const uint32_t p = row0 / kPanelRows, R = panel_rows(n, p);
+
+  // x first: its staging barrier is the longer wait
+  const uint32_t pieces = K * sizeof(XT) / 16;
+  const rsrc_t xr = make_rsrc((const void *)x_, K * sizeof(XT));
+  u32x4 xv0 = {}, xv1 = {};
+  const uint32_t i0 = threadIdx.x, i1 = threadIdx.x + threads;
+  if (i0 < pieces) xv0 = __builtin_amdgcn_raw_buffer_load_b128(xr, i0 * 16, 0, 0);
+  if (i1 < pieces) xv1 = __builtin_amdgcn_raw_buffer_load_b128(xr, i1 * 16, 0, 0);
+
+  // lane (u, r8): unit (j, h) = (u / 2 % 2, u % 2) of chunk 2 pair + u / 4,
+  // row r8 of each group.  Rows past a partial panel's last read row R - 1
+  // (never stored).
+  const uint32_t u = lane >> 3, cp = u >> 2, j = (u >> 1) & 1, h = u & 1;
+  const rsrc_t wq = make_rsrc((const void *)qs_, n * K), ws = make_rsrc((const void *)sc_, n * (K / 32) * 2);
+  const rsrc_t wz = make_rsrc((const void *)qs_, 0);
+  uint32_t w_voff[NR], s_voff[NR];
+#pragma unroll
+  for (int g = 0; g < NR; ++g) {
+    const uint32_t want = row0 % kPanelRows + 8 * g + (lane & 7), r = want < R ? want : R - 1;
+    w_voff[g] = cp * R * kChunkK + ((2 * j + h) * R + r) * 16;
+    s_voff[g] = cp * R * 4 + (h * R + r) * 2;
+  }
+  // Pairs past the range load through an empty resource and the missing
+  // second chunk of an odd last pair at an offset outside the range.
+  PairW<NR> win[WIN];
+  auto load = [&](PairW<NR> &b, uint32_t pr) {
+    const bool in = pr < pairs, none = 2 * pr + cp >= chunks;
+    const uint32_t so = (uint32_t)panel_chunk_qs(K, p, R, 2 * pr);
+    const uint32_t ss = (uint32_t)panel_chunk_sc(K, p, R, 2 * pr) * 2;
+#pragma unroll
+    for (int g = 0; g < NR; ++g) {
+      b.w[g] = __builtin_amdgcn_raw_buffer_load_b128(in ? wq : wz, none ? kNowhere : w_voff[g], so, 0);
+      b.s[g] = __builtin_amdgcn_raw_buffer_load_b16(in ? ws : wz, none ? kNowhere : s_voff[g], ss, 0);
+    }
+  };
+#pragma unroll
+  for (int k = 0; k < WIN; ++k) load(win[k], wave + k * waves);
+
+  const uint32_t erow = row0 + threadIdx.x;
+  const bool mine = threadIdx.x < kRows && erow < n;
+  const RowEpi epi = epi_load<MODE>(mine, erow, K, (const gfloat *)out_, (const gfloat *)bias_,
+                                    (const gfloat *)vb_, (const guint *)pos_);
+
+  for (uint32_t i = threadIdx.x; i < pieces; i += threads) {
+    const u32x4 v =
+        i == i0 ? xv0 : (i == i1 ? xv1 : __builtin_amdgcn_raw_buffer_load_b128(xr, i * 16, 0, 0));
+    reinterpret_cast<u32x4 *>(xs)[i] = v;
+  }
+  __syncthreads();
+
+  float acc[NR];
+#pragma unroll
+  for (int g = 0; g < NR; ++g) acc[g] = 0.0f;
+#pragma unroll 1
+  for (uint32_t base = wave;;) {
+    // the window's x is read while its weights are in flight (a missing chunk
+    // reads the last one's, and its sum is dropped)
+    XUnitOf<XT> xu[WIN];
+#pragma unroll
+    for (int k = 0; k < WIN; ++k) {
+      const uint32_t want = 2 * (base + k * waves) + cp, c = want < chunks ? want : chunks - 1;
+      read_x(xu[k], xs + c * kChunkK + h * 32 + j * 16);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < WIN; ++k) {
+      const bool real = 2 * (base + k * waves) + cp < chunks;
+#pragma unroll
+      for (int g = 0; g < NR; ++g) {
+        const float sum = __builtin_fmaf(xunit_dot(win[k].w[g], xu[k].v),
+                                         (float)__builtin_bit_cast(f16, (uint16_t)win[k].s[g]), acc[g]);
+        acc[g] = real ? sum : acc[g];
+      }
+      if constexpr (!ONE) {
+        load(win[k], base + (k + WIN) * waves);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if constexpr (ONE) break;
+    base += WIN * waves;
+    if (base >= pairs) break;
+  }
+#pragma unroll
+  for (int g = 0; g < NR; ++g) {
+    const float v = sum_units(acc[g]);
+    if (lane < 8) red[wave * kRows + 8 * g + lane] = v;
+  }
+  __syncthreads();
+  if (!mine) return;
+  float v = red[threadIdx.x];  // the waves' partials in wave order
+  for (uint32_t w = 1; w < waves; ++w) v += red[w * kRows + threadIdx.x];
+  epi_store<MODE>(v, epi, erow, K, (gfloat *)out_, (gfloat *)kc_, (gfloat *)vc_);
+}
+
+// 48 bytes of arguments; the QKV mode's four more in a kernel of its own.
+template <typename XT, int MODE, int NR, int WIN, bool ONE>
+__global__ __launch_bounds__(kRowWaves * 64) void q8_gemv_rows_kernel(uint64_t x, uint64_t qs, uint32_t n,
+                                                                      uint32_t K, uint64_t sc, uint64_t out,
+                                                                      uint64_t bias) {
+  gemv_rows<XT, MODE, NR, WIN, ONE>(x, qs, n, K, sc, out, bias, 0, 0, 0, 0);
+}
+template <typename XT, int NR, int WIN, bool ONE>
+__global__ __launch_bounds__(kRowWaves * 64) void q8_gemv_rows_qkv_kernel(
+    uint64_t x, uint64_t qs, uint32_t n, uint32_t K, uint64_t sc, uint64_t out, uint64_t qb, uint64_t vb,
+    uint64_t kc, uint64_t vc, uint64_t pos) {
+  gemv_rows<XT, kQkv, NR, WIN, ONE>(x, qs, n, K, sc, out, qb, vb, kc, vc, pos);
+}
+
+template <typename XT, int MODE, int NR, int WIN, bool ONE>
+void launch_rows(const GemvArgs &a) {
+  const uint32_t pairs = (a.k / kChunkK + 1) / 2, waves = ONE ? (pairs + WIN - 1) / WIN : kRowWaves;
+  const dim3 grid((a.n + 8 * NR - 1) / (8 * NR)), block(waves * 64);
+  const size_t lds = a.k * sizeof(XT) + waves * 8 * NR * 4;
+  if constexpr (MODE == kQkv)
+    hipLaunchKernelGGL((q8_gemv_rows_qkv_kernel<XT, NR, WIN, ONE>), grid, block, lds, stream(), addr(a.x),
+                       addr(a.qs), a.n, a.k, addr(a.sc), addr(a.out), addr(a.qb), addr(a.vb), addr(a.kc),
+                       addr(a.vc), addr(a.pos));
+  else
+    hipLaunchKernelGGL((q8_gemv_rows_kernel<XT, MODE, NR, WIN, ONE>), grid, block, lds, stream(), addr(a.x),
+                       addr(a.qs), a.n, a.k, addr(a.sc), addr(a.out), addr(a.bias));
+}
+
+// Rows per workgroup: 8 while that is at most one workgroup per CU or so,
+// else 16, which halve the x staged per weight (issued from C, us, 8 / 16 /
+// 32 rows: 1280 x 1280 2.5 / 2.7 / -, 3840 x 1280 4.1 / 2.7 / 3.1, 5120 x
+// 1280 5.5 / 3.0 / 3.3, 1280 x 5120 3.6 / 4.5 / -).  One pair of chunks per
+// wave up to K = 2048; three, all in flight at once, above (1280 x 1280 with
+// two or three per wave 2.8); past 6144 sixteen waves go round.
+constexpr uint32_t kRows8 = 2304;
+template <typename XT, int MODE, int NR>
+void pick_rows(const GemvArgs &a) {
+  const uint32_t pairs = (a.k / kChunkK + 1) / 2;
+  if (pairs <= kRowWaves) launch_rows<XT, MODE, NR, 1, true>(a);
+  else if (pairs <= 3 * kRowWaves) launch_rows<XT, MODE, NR, 3, true>(a);
+  else launch_rows<XT, MODE, NR, 3, false>(a);
 }
 
 template <typename XT, int MODE>
@@ -432,26 +602,15 @@ int launch(const char *what, const GemvArgs &a) {
   } else if (int rc = deferred_before_write(a.out, (size_t)a.n * 4)) {
     return rc;
   }
-  const uint32_t np = (a.n + kPanelRows - 1) / kPanelRows, C = a.k / kChunkK;
-  // Few panels and a long K (the 5120-wide FFN down projection: 40 panels)
-  // leave most CUs idle and each wave with a long chain of loads: split K
-  // over up to four workgroups per panel, >= 16 chunks each.
-  GemvArgs b = a;
-  b.splits = 1;
-  if (np < 128 && C >= 32) {
-    b.splits = C / 16 < 4 ? C / 16 : 4;
-    if (int rc = workspace((size_t)np * b.splits * 32 * 4, np, &b.ws, &b.cnt)) return rc;
-  }
+  const uint32_t np = (a.n + kPanelRows - 1) / kPanelRows;
   if (np >= kWidePanels)
-    hipLaunchKernelGGL((q8_gemv_kernel<XT, MODE, kWaves>), dim3(np, b.splits), dim3(kWaves * 64),
-                       (lds_bytes<XT, kWaves>(a.k)), stream(), b.qs, b.sc, b.x, b.n, b.k,
-                       C / b.splits, C % b.splits, b.out, b.bias, b.ws, b.cnt, b.qb, b.vb, b.kc,
-                       b.vc, b.pos);
+    hipLaunchKernelGGL((q8_gemv_kernel<XT, MODE>), dim3(np), dim3(kWaves * 64), lds_bytes<XT>(a.k), stream(),
+                       addr(a.qs), addr(a.sc), addr(a.x), a.n, a.k, addr(a.out),
+                       addr(MODE == kQkv ? a.qb : a.bias), addr(a.vb), addr(a.kc), addr(a.vc), addr(a.pos));
+  else if (a.n > kRows8)
+    pick_rows<XT, MODE, 2>(a);
   else
-    hipLaunchKernelGGL((q8_gemv_kernel<XT, MODE, kWavesNarrow>), dim3(np, b.splits),
-                       dim3(kWavesNarrow * 64), (lds_bytes<XT, kWavesNarrow>(a.k)), stream(), b.qs,
-                       b.sc, b.x, b.n, b.k, C / b.splits, C % b.splits, b.out, b.bias, b.ws, b.cnt,
-                       b.qb, b.vb, b.kc, b.vc, b.pos);
+    pick_rows<XT, MODE, 1>(a);
   return check_launch(what);
 }
 
