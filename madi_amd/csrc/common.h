@@ -22,6 +22,8 @@ int cu_count();
 // Grows on demand (a grow waits for the device; an outgrown buffer is kept,
 // not freed, because graphs captured earlier still name it); all of them are
 // freed by madi_cleanup.
+// The counters come first, kWorkspaceCounterBytes of them, then the partials.
+constexpr size_t kWorkspaceCounterBytes = 16384 * 4;
 int workspace(size_t partial_bytes, size_t counters, float **partials, uint32_t **cnt);
 // The same for a caller that has another way: false, with no error recorded,
 // where the workspace cannot grow (a graph capture, no memory).

@@ -21,7 +21,7 @@ hipStream_t g_stream = nullptr;
 // Orders a newly chosen stream after the work already issued on the old one.
 hipEvent_t g_switch = nullptr;
 // Split-K workspace: kCounters zeroed arrival counters, then the partial sums.
-constexpr size_t kCounters = 16384;
+constexpr size_t kCounters = kWorkspaceCounterBytes / 4;
 void *g_ws = nullptr;
 size_t g_ws_bytes = 0;
 // Workspaces outgrown by a larger split shape.  A HIP graph captured before

@@ -12,6 +12,9 @@
 // one rounding the pipeline adds after the product, dropped: it only moves
 // the result away from the fp32 reference of test_batchproj.zig:72-78).
 //
+// Few rows on narrow weights run q8_skinny16_kernel (below), a workgroup per
+// 16 weight rows; the rest q8_skinny_kernel.
+//
 // Workgroup: P weight panels (32 rows each; P = 4 for the 51866-row vocab
 // matrix from 9 rows, 2 for narrow weights at prefill sizes (panel pairs),
 // 1 otherwise) x one slice of 32 activation rows (the MFMA columns), KW
@@ -40,6 +43,10 @@ namespace {
 
 constexpr uint32_t kSlice = 32;  // activation rows per workgroup (MFMA columns)
 
+typedef __attribute__((address_space(1))) float gfloat;
+typedef __attribute__((address_space(1))) f16 gf16;
+typedef __attribute__((address_space(1))) f16x2 gf16x2;
+typedef __attribute__((address_space(1))) f16x4 gf16x4;
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 __device__ inline rsrc_t make_rsrc(const void *base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
@@ -207,16 +214,22 @@ constexpr int skinny_lds() {
 //
 // Grid (x, y, z) = (panel group, 32-row activation slice, K split).  The
 // arguments are scalars in the order the kernel first needs them, so the
-// leading ones arrive preloaded in SGPRs, and the set-up has no integer
-// division: split s covers chunks [s * cper + min(s, crem), + cper + (s <
-// crem)).  `x`, `out`: f32 [m][k], [m][n], or with H f16 [m][k], [m][n] (the
-// sum rounded once to f16); `ws`, `cnt`: partial tiles and arrival counters
-// (zero between uses) when K is split.
+// leading ones arrive preloaded in SGPRs, pointers among them as integers (the
+// runtime looks pointer arguments up, 0.09 us each on the host) and 64 bytes
+// in all, and the set-up has no integer division: split s covers chunks [s *
+// cper + min(s, crem), + cper + (s < crem)).  `x`, `out`: f32 [m][k], [m][n],
+// or with H f16 [m][k], [m][n] (the sum rounded once to f16); `ws`: the
+// library's workspace, arrival counters (zero between uses) and partial
+// tiles, when K is split.
 template <int P, int KW, int XR, int WIN, bool H = false>
 __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(KW / 4 > 2 ? KW / 4 : 2))) void q8_skinny_kernel(
-    const uint8_t *__restrict__ qs, const f16 *__restrict__ sc, const void *__restrict__ x,
-    uint32_t M, uint32_t N, uint32_t K, uint32_t cper, uint32_t crem, uint32_t groups,
-    void *__restrict__ out, f32x4 *ws, uint32_t *cnt) {
+    uint64_t qs_, uint64_t sc_, uint64_t x_, uint32_t M, uint32_t N, uint32_t K, uint32_t cper,
+    uint32_t groups, uint32_t splits, uint64_t out_, uint64_t ws_) {
+  const uint8_t *qs = (const uint8_t *)qs_;
+  const f16 *sc = (const f16 *)sc_;
+  const void *x = (const void *)x_;
+  const uint32_t crem = K / kChunkK - cper * splits;
+  const uint32_t slices = (M + kSlice - 1) / kSlice;
   __shared__ __attribute__((aligned(16))) uint8_t smem[skinny_lds<P, KW, XR, WIN, H>()];
 
   // Consecutive workgroups go to different XCDs (round-robin, x fastest).
@@ -224,7 +237,6 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(KW / 4 
   // panel group g runs on XCD g % 8 and shares its weights in that L2.
   const uint32_t grp = blockIdx.x, slice = blockIdx.y, split = blockIdx.z;
   if (grp >= groups) return;
-  const uint32_t splits = gridDim.z;
 
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -337,9 +349,11 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(KW / 4 
     // the splits' partials in split order and stores the rows.
     __shared__ uint32_t arrived;
     constexpr int kSc1 = 16;
-    const uint32_t tile = grp * gridDim.y + slice;
+    const uint32_t tile = grp * slices + slice;
+    typedef __attribute__((address_space(1))) uint32_t guint;
+    guint *cnt = (guint *)ws_;
     const uint32_t part = P * 4 * 64 * 16;  // bytes per partial tile
-    const __amdgpu_buffer_rsrc_t wsr = make_rsrc(ws, groups * gridDim.y * splits * part);
+    const __amdgpu_buffer_rsrc_t wsr = make_rsrc((const uint8_t *)ws_ + kWorkspaceCounterBytes, groups * slices * splits * part);
     if (wave < 4) {
 #pragma unroll
       for (int t = 0; t < P; ++t)
@@ -374,16 +388,16 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(KW / 4 
     if (grp * P + t >= np) break;
     const uint32_t R = pl.R[t];
     if constexpr (H) {
-      f16 *o = static_cast<f16 *>(out) + (size_t)m * N + pl.p[t] * kPanelRows + nl;
+      gf16 *o = (gf16 *)out_ + (size_t)m * N + pl.p[t] * kPanelRows + nl;
       const f16x4 hv = {(f16)v[t].x, (f16)v[t].y, (f16)v[t].z, (f16)v[t].w};
       if (nl + 4 <= R) {
         // o is 8-byte aligned when N % 4 == 0 and 4-byte aligned when N is
         // even (out is 16-byte aligned and 32 p + nl is a multiple of 4)
         if (N % 4 == 0) {
-          *reinterpret_cast<f16x4 *>(o) = hv;
+          *(gf16x4 *)o = hv;
         } else if (N % 2 == 0) {
-          reinterpret_cast<f16x2 *>(o)[0] = (f16x2){hv.x, hv.y};
-          reinterpret_cast<f16x2 *>(o)[1] = (f16x2){hv.z, hv.w};
+          ((gf16x2 *)o)[0] = (f16x2){hv.x, hv.y};
+          ((gf16x2 *)o)[1] = (f16x2){hv.z, hv.w};
         } else {
           o[0] = hv.x;
           o[1] = hv.y;
@@ -397,7 +411,7 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(KW / 4 
       }
       continue;
     }
-    float *o = static_cast<float *>(out) + (size_t)m * N + pl.p[t] * kPanelRows + nl;
+    gfloat *o = (gfloat *)out_ + (size_t)m * N + pl.p[t] * kPanelRows + nl;
     if (nl + 4 <= R) {
       o[0] = v[t].x;
       o[1] = v[t].y;
@@ -409,6 +423,173 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(KW / 4 
       if (nl + 2 < R) o[2] = v[t].z;
     }
   }
+}
+
+// One projection: out[m][n] = sum_k x[m][k] w[n][k]; x and out f32, or f16
+// for the launches with H set.
+struct Proj {
+  void *out;
+  const void *x;
+  const uint8_t *qs;
+  const f16 *sc;
+  uint32_t m, n, k;
+  const char *what;
+};
+
+// ---- narrow matrices (the decoder's projections): a workgroup per 16 weight
+// rows with all of K.
+//
+// v_mfma_f32_16x16x32_f16 with 16 weight rows and 16 activation rows: lane
+// (g, c) loads unit (j, h) = (g % 2, g / 2) of row c per chunk (four 256-byte
+// runs per instruction), which dequantises to its fragments of both 32-wide
+// steps (step e: k = 16g + 8e .. + 8).  Two chunks in flight per wave and up
+// to twelve waves, so a K of 1280 is one round of loads; 80 workgroups for
+// 1280 rows where the panel kernel below has 40, and a K of 5120 meets in LDS
+// instead of through memory.
+constexpr int kRowsWin = 2;  // (the sums below name both slots)
+constexpr uint32_t kRowsWaves = 12;
+template <int XR, bool ONE>
+__global__ __launch_bounds__(1024) void q8_skinny16_kernel(uint64_t x_, uint64_t qs_, uint32_t M, uint32_t N,
+                                                           uint32_t K, uint32_t waves, uint64_t sc_,
+                                                           uint64_t out_) {
+  constexpr int T = XR > 16 ? 2 : 1, WIN = kRowsWin;  // 16-row activation tiles
+  extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t g = lane >> 4, c16 = lane & 15;
+  const uint32_t row0 = blockIdx.x * 16, p = row0 / kPanelRows, R = panel_rows(N, p);
+  const uint32_t chunks = K / kChunkK;
+  const uint32_t m0 = blockIdx.y * kSlice, rows = M - m0 < kSlice ? M - m0 : kSlice;
+  const rsrc_t xr = make_rsrc((const uint8_t *)x_ + (size_t)m0 * K * 4, rows * K * 4);
+  const rsrc_t wq = make_rsrc((const void *)qs_, N * K), ws = make_rsrc((const void *)sc_, N * (K / 32) * 2);
+  const rsrc_t wz = make_rsrc((const void *)qs_, 0);
+  const uint32_t x_voff = (lane >> 4) * K * 4 + (lane & 15) * 16;
+  const uint32_t want = row0 % kPanelRows + c16, r = want < R ? want : R - 1;
+  const uint32_t w_voff = ((2 * (g & 1) + (g >> 1)) * R + r) * 16, s_voff = ((g >> 1) * R + r) * 2;
+  // piece j = 2g + e of an activation row is kept as piece 4e + g, which
+  // spreads the fragment reads of two lane groups over all banks
+  auto tile_piece = [](uint32_t row, uint32_t j) { return x_piece(row, (j & 1) * 4 + (j >> 1)); };
+
+  struct Slot {
+    u32x4 w;
+    uint32_t s;
+    f32x4 x[XR / 4];
+  } win[WIN];
+  auto load_x = [&](Slot &b, uint32_t c) {
+#pragma unroll
+    for (int i = 0; i < XR / 4; ++i)
+      b.x[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                             c < chunks ? xr : wz, x_voff + i * 16 * K, c * kChunkK * 4, 0));
+  };
+  auto load_w = [&](Slot &b, uint32_t c) {
+    const bool in = c < chunks;
+    b.w = __builtin_amdgcn_raw_buffer_load_b128(in ? wq : wz, w_voff, (uint32_t)panel_chunk_qs(K, p, R, c), 0);
+    b.s = __builtin_amdgcn_raw_buffer_load_b16(in ? ws : wz, s_voff, (uint32_t)panel_chunk_sc(K, p, R, c) * 2, 0);
+  };
+#pragma unroll
+  for (int k = 0; k < WIN; ++k) load_x(win[k], wave + k * waves);
+#pragma unroll
+  for (int k = 0; k < WIN; ++k) load_w(win[k], wave + k * waves);
+
+  uint8_t *xt = dyn + wave * (WIN * XR * 128);
+  // a sum of its own per window slot and step: short chains, added in pairs
+  f32x4 acc[T][WIN][2];
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int k = 0; k < WIN; ++k) acc[t][k][0] = acc[t][k][1] = (f32x4){};
+#pragma unroll 1
+  for (uint32_t base = wave;;) {
+    f16x8 xf[WIN][T][2];
+#pragma unroll
+    for (int k = 0; k < WIN; ++k) {
+      uint8_t *tile = xt + k * (XR * 128);
+#pragma unroll
+      for (int i = 0; i < XR / 4; ++i) {
+        const uint32_t row = 4 * i + (lane >> 4), k4 = lane & 15;
+        const f32x4 v = win[k].x[i];
+        *reinterpret_cast<f16x4 *>(tile + tile_piece(row, k4 >> 1) + (k4 & 1) * 8) =
+            (f16x4){(f16)v.x, (f16)v.y, (f16)v.z, (f16)v.w};
+      }
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          xf[k][t][e] = (f16x8){};
+          if (XR >= 16 || c16 < XR)
+            xf[k][t][e] = *reinterpret_cast<const f16x8 *>(tile + tile_piece(16 * t + c16, 2 * g + e));
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // slots past the range hold zero weights and zero activations
+#pragma unroll
+    for (int k = 0; k < WIN; ++k) {
+      f16x8 lo, hi;
+      dequant16(win[k].w, __builtin_bit_cast(f16, (uint16_t)win[k].s), lo, hi);
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        acc[t][k][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, xf[k][t][0], acc[t][k][0], 0, 0, 0);
+        acc[t][k][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, xf[k][t][1], acc[t][k][1], 0, 0, 0);
+      }
+      if constexpr (!ONE) {
+        load_x(win[k], base + (k + WIN) * waves);
+        load_w(win[k], base + (k + WIN) * waves);
+      }
+    }
+    if constexpr (ONE) break;
+    base += WIN * waves;
+    if (base >= chunks) break;
+  }
+  __syncthreads();  // every wave is done with its activation tiles
+  // lane (g, c) holds weight rows 4g .. + 3 of activation row 16t + c
+  float *red = reinterpret_cast<float *>(dyn);  // [wave][t][lane][4]
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+    *reinterpret_cast<f32x4 *>(red + ((wave * T + t) * 64 + lane) * 4) =
+        (acc[t][0][0] + acc[t][0][1]) + (acc[t][1][0] + acc[t][1][1]);
+  __syncthreads();
+  gfloat *out = (gfloat *)out_;
+  for (uint32_t i = threadIdx.x; i < 256 * T; i += waves * 64) {
+    const uint32_t n = i & 15, m = i >> 4;
+    const float *v = red + ((m >> 4) * 64 + (n >> 2) * 16 + (m & 15)) * 4 + (n & 3);
+    // the waves' partials, two sums
+    float sum = v[0], odd = waves & 1 ? 0.0f : v[(waves - 1) * (T * 256)];
+    for (uint32_t w = 1; w + 1 < waves; w += 2) {
+      odd += v[w * (T * 256)];
+      sum += v[(w + 1) * (T * 256)];
+    }
+    sum += odd;
+    if (row0 + n < N && m < rows) out[(size_t)(m0 + m) * N + row0 + n] = sum;
+  }
+}
+
+template <int XR>
+int launch_skinny16(const Proj &a) {
+  constexpr uint32_t kSlot = kRowsWin * XR * 128, kPart = (XR > 16 ? 2 : 1) * 1024;
+  static_assert(kSlot >= kPart, "the partials fit the activation tiles");
+  const uint32_t want = (a.k / kChunkK + kRowsWin - 1) / kRowsWin;
+  const uint32_t waves = want < kRowsWaves ? want : kRowsWaves;
+  const dim3 grid((a.n + 15) / 16, (a.m + kSlice - 1) / kSlice);
+  const auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(waves * 64), waves * kSlot, stream(), (uint64_t)a.x, (uint64_t)a.qs,
+                       a.m, a.n, a.k, waves, (uint64_t)a.sc, (uint64_t)a.out);
+  };
+  if (want <= kRowsWaves) go(q8_skinny16_kernel<XR, true>);
+  else go(q8_skinny16_kernel<XR, false>);
+  return check_launch(a.what);
+}
+
+// Where a workgroup per 16 rows pays (issued from C, us, 32-row panels / 16
+// rows): while it is at most one workgroup per CU, 1280 x 1280 at 8 / 16 / 32
+// / 64 rows 3.35 / 2.64, 3.75 / 2.88, 4.42 / 3.72, 4.48 / 3.88, 3840 x 1280 at
+// 8 / 16 / 32 rows 3.43 / 2.92, 3.87 / 3.19, 4.51 / 4.17; past that the
+// activations, which every workgroup loads, cost more (5120 x 1280 at 8 / 32
+// rows 3.47 / 3.53, 4.6 / 5.7, 2560 x 1280 at 64 4.5 / 5.4).  A long K on few
+// panels, which the panel kernel splits over workgroups that meet through
+// memory, only up to 8 rows (1280 x 5120 at 8 / 16 rows 6.11 / 4.83, 6.5 / 6.9).
+bool skinny16_suits(uint32_t m, uint32_t n, uint32_t k) {
+  const uint64_t wgs = (uint64_t)((n + 15) / 16) * ((m + kSlice - 1) / kSlice);
+  return wgs <= (uint64_t)cu_count() && (k <= 2048 || (m <= 8 && n < 128 * kPanelRows));
 }
 
 // Launch shapes.  Single panels (decoder projections, 40 - 160 panels): eight
@@ -432,17 +613,6 @@ constexpr int kGroupWaves = 4, kGroupWin = 2;
 constexpr int kPairWaves = 4, kPairWin = 2;
 constexpr uint32_t kMaxSplits = 4;
 
-// One projection: out[m][n] = sum_k x[m][k] w[n][k]; x and out f32, or f16
-// for the launches with H set.
-struct Proj {
-  void *out;
-  const void *x;
-  const uint8_t *qs;
-  const f16 *sc;
-  uint32_t m, n, k;
-  const char *what;
-};
-
 template <int P, int KW, int XR, int WIN, bool H = false>
 int launch_skinny(const Proj &a) {
   const uint32_t np = (a.n + kPanelRows - 1) / kPanelRows;
@@ -451,18 +621,17 @@ int launch_skinny(const Proj &a) {
   // Few panels and a long K (the FFN down projection, 40 panels x 80 chunks):
   // split K over up to four workgroups per tile, >= 16 chunks each.
   uint32_t splits = 1;
-  f32x4 *ws = nullptr;
-  uint32_t *cnt = nullptr;
+  uint32_t *cnt = nullptr;  // the workspace: counters, then partials
   if (P == 1 && np < 128 && C >= 32) {
     splits = C / 16 < kMaxSplits ? C / 16 : kMaxSplits;
     float *w = nullptr;
     const size_t part = (size_t)P * 4 * 64 * 16;
     if (int rc = workspace(groups * slices * splits * part, groups * slices, &w, &cnt)) return rc;
-    ws = reinterpret_cast<f32x4 *>(w);
   }
   const dim3 grid((groups + 7) / 8 * 8, slices, splits);
-  hipLaunchKernelGGL((q8_skinny_kernel<P, KW, XR, WIN, H>), grid, dim3(KW * 64), 0, stream(), a.qs,
-                     a.sc, a.x, a.m, a.n, a.k, C / splits, C % splits, groups, a.out, ws, cnt);
+  hipLaunchKernelGGL((q8_skinny_kernel<P, KW, XR, WIN, H>), grid, dim3(KW * 64), 0, stream(), (uint64_t)a.qs,
+                     (uint64_t)a.sc, (uint64_t)a.x, a.m, a.n, a.k, C / splits, groups, splits, (uint64_t)a.out,
+                     (uint64_t)cnt);
   return check_launch(a.what);
 }
 
@@ -516,6 +685,12 @@ extern "C" int madi_q8_pproj(float *out, const float *in, const void *qs, const 
   // while that fits (M = 224 / 288 / 320: 5.6 / 5.8 / 5.9 us against 8.0 on
   // the GEMM's 32 x 128 tiles, which leave 156 CUs idle), and only then the
   // GEMM.
+  if (skinny16_suits(m, n, k)) {
+    const Proj a{out, in, static_cast<const uint8_t *>(qs), static_cast<const f16 *>(scales), m, n,
+                 k, "madi_q8_pproj"};
+    if (m <= 8) return launch_skinny16<8>(a);
+    return m <= 16 ? launch_skinny16<16>(a) : launch_skinny16<32>(a);
+  }
   const uint64_t np = (n + kPanelRows - 1) / kPanelRows, slices = (m + kSlice - 1) / kSlice;
   const uint64_t skinny_wgs = np * slices, cus = (uint64_t)cu_count();
   if (m > kSlice && n < 2048 && k < 4096 && skinny_wgs > cus && (np + 1) / 2 * slices <= cus) {
