@@ -108,6 +108,36 @@ def check(rc: int, what: str) -> None:
         raise MadiError(rc, what, last_error())
 
 
+_LETTER = {_P: "p", _U32: "i", _I: "i", ctypes.c_float: "f"}
+
+
+def _fail(code: int, name: str):
+    raise MadiError(code, name, last_error())
+
+
+class _Calls:
+    """The entry points as C callables (csrc/pycall.c), bound at first use:
+    calls.madi_q8_gemv(out, x, qs, ...) takes tensors, integers or None for
+    pointers and raises MadiError on a nonzero code.  Through ctypes and a
+    wrapper's data_ptr() calls a projection cost about 0.9 us of host time
+    beside the launch's 2.8; this costs 0.3."""
+
+    def __getattr__(self, name: str):
+        if name not in SIGNATURES or SIGNATURES[name][0] is not _I:
+            raise AttributeError(name)
+        fn = getattr(lib(), name)
+        sig = "".join(_LETTER.get(t, "?") for t in SIGNATURES[name][1])
+        try:
+            from . import _pycall
+        except ImportError as e:
+            raise ImportError(f"{e}: build it with `python -m madi_amd.build`") from e
+        bound = _pycall.bind(ctypes.cast(fn, _P).value, sig, name, _fail)
+        setattr(self, name, bound)
+        return bound
+
+
+calls = _Calls()
+
 _FNS: dict = {}
 
 

@@ -10,6 +10,7 @@ import concurrent.futures
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -56,6 +57,19 @@ def build_issue(lib: str = LIB, out: str = ISSUE_LIB) -> str:
     return out
 
 
+PYCALL_SRC = os.path.join(CSRC, "pycall.c")
+PYCALL_LIB = os.path.join(HERE, "_pycall" + sysconfig.get_config_var("EXT_SUFFIX"))
+
+
+def build_pycall(out: str = PYCALL_LIB) -> str:
+    """The wrappers' call path (csrc/pycall.c), a CPython extension module."""
+    tmp = out + ".tmp"
+    _run(["gcc", "-O2", "-std=c11", "-shared", "-fPIC", "-Wall", "-I",
+          sysconfig.get_paths()["include"], PYCALL_SRC, "-o", tmp])
+    os.replace(tmp, out)
+    return out
+
+
 def _run(cmd):
     r = subprocess.run(cmd, capture_output=True, text=True)
     err = "\n".join(l for l in r.stderr.splitlines() if "packed-fp32-ops" not in l)
@@ -85,6 +99,7 @@ def build(verbose: bool = False, extra_flags=(), out: str = LIB, obj_dir: str = 
     os.replace(tmp, out)
     if out == LIB:
         build_issue()
+        build_pycall()
     return out
 
 

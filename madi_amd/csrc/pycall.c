@@ -9,11 +9,14 @@
  *
  * Through ctypes a decoder projection's call spent about as long in argument
  * conversion as in the HIP launch, and short kernels waited for the host
- * (one 1280 x 1280 GEMV with bias 4.6 us a call from Python on a kernel of
- * 2.9-3.9 us). */
+ * (a 64 x 64 GEMV with bias: 3.55 us a call through ctypes
+ * with the pointers at hand, 3.11 through the whole wrapper now, 2.8 of it
+ * the launch). */
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
+#include <stddef.h>
 #include <stdint.h>
+#include <string.h>
 
 #define MAX_INTS 10
 #define MAX_FLOATS 2
@@ -29,13 +32,9 @@ typedef struct {
 
 static PyObject *s_data_ptr;
 
-/* An int's value modulo 2^64, as ctypes takes it for a pointer or a 32-bit
- * argument (the callee reads the low half). */
+/* An integer's value modulo 2^64, as ctypes takes it (anything with
+ * __index__; the callee of a 32-bit argument reads the low half). */
 static int as_int(PyObject *o, uint64_t *v) {
-  if (!PyLong_Check(o)) {
-    PyErr_Format(PyExc_TypeError, "int expected instead of %.100s", Py_TYPE(o)->tp_name);
-    return -1;
-  }
   *v = PyLong_AsUnsignedLongLongMask(o);
   return *v == (uint64_t)-1 && PyErr_Occurred() ? -1 : 0;
 }

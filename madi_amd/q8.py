@@ -14,7 +14,7 @@ from dataclasses import dataclass
 
 import numpy as np
 
-from ._lib import EPI_BIAS, EPI_BIAS_GELU, EPI_BIAS_RES, EPI_NONE, MadiError, call, check, lib
+from ._lib import EPI_BIAS, EPI_BIAS_GELU, EPI_BIAS_RES, EPI_NONE, MadiError, call, calls, check, lib
 
 D = 1280          # encoder.zig:12, decoder.zig:12
 MLP = 5120        # encoder.zig:15
@@ -55,6 +55,8 @@ def getFunction(name: str) -> int:
 
 
 def _fn(f) -> int:
+    if type(f) is int:
+        return f
     return getFunction(f) if isinstance(f, str) else int(f)
 
 
@@ -180,7 +182,7 @@ def quantize(w16, n: int, k: int, device="cuda") -> Q8:
     import torch
     dq = torch.empty(n * k, dtype=torch.uint8, device=device)
     ds = torch.empty(n * (k // 32), dtype=torch.int16, device=device)
-    call("madi_q8_quantize", dq.data_ptr(), ds.data_ptr(), ptr(w16), n, k)
+    calls.madi_q8_quantize(dq, ds, w16, n, k)
     return Q8(dq.data_ptr(), ds.data_ptr(), (dq, ds))
 
 
@@ -200,7 +202,7 @@ def kDeq(wdq, w: Q8, n: int, k: int) -> None:
     """encoder.zig:154-159: Q8 [N][K] -> F16 [K][N] (dequant_q8_f16).  Deferred:
     an F16 GEMM on wdq runs the fused Q8 kernel; materialize(wdq) before reading
     wdq outside the library."""
-    call("madi_q8_dequant_f16", ptr(wdq), w.qs, w.scales, n, k)
+    calls.madi_q8_dequant_f16(wdq, w.qs, w.scales, n, k)
 
 
 def deqW16(wdq, w: Q8, n: int, k: int) -> None:
@@ -210,26 +212,25 @@ def deqW16(wdq, w: Q8, n: int, k: int) -> None:
 
 def kGemmQ8(a, w: Q8, c, m: int, n: int, k: int) -> None:
     """Fused kDeq + kM4 (encoder.zig:125-130, 154-159): C = A . deq(W)^T, f16."""
-    call("madi_q8_gemm", ptr(a), w.qs, w.scales, ptr(c), None, m, n, k, EPI_NONE)
+    calls.madi_q8_gemm(a, w.qs, w.scales, c, None, m, n, k, EPI_NONE)
 
 
 def kGemmQ8Bias(a, w: Q8, c, bias, m: int, n: int, k: int, gelu: bool = False) -> None:
     """Fused kDeq + kM4Bias (encoder.zig:131-136) with the m4_gemm_bias or
     m4_gemm_bias_gelu epilogue (m4_gemm.metal:60-115)."""
-    call("madi_q8_gemm", ptr(a), w.qs, w.scales, ptr(c), ptr(bias), m, n, k,
-         EPI_BIAS_GELU if gelu else EPI_BIAS)
+    calls.madi_q8_gemm(a, w.qs, w.scales, c, bias, m, n, k, EPI_BIAS_GELU if gelu else EPI_BIAS)
 
 
 def kM4(f, a, b, c, m: int, n: int, k: int) -> None:
     """encoder.zig:125-130: C = A . B, f16 [M][K] . [K][N], f = the m4_gemm_nn
     handle (or its name).  b is an F16 weight or the wdq a kDeq just recorded
     (then the fused Q8 GEMM runs)."""
-    call("madi_m4_gemm", _fn(f), ptr(a), ptr(b), ptr(c), None, m, n, k)
+    calls.madi_m4_gemm(_fn(f), a, b, c, None, m, n, k)
 
 
 def kM4Bias(f, a, b, c, bias, m: int, n: int, k: int) -> None:
     """encoder.zig:131-136, f = the m4_gemm_bias or m4_gemm_bias_gelu handle."""
-    call("madi_m4_gemm", _fn(f), ptr(a), ptr(b), ptr(c), ptr(bias), m, n, k)
+    calls.madi_m4_gemm(_fn(f), a, b, c, bias, m, n, k)
 
 
 def kFlash(f, out, q, k, v, seq: int, nh: int = NH) -> None:
@@ -242,7 +243,7 @@ def kFlash(f, out, q, k, v, seq: int, nh: int = NH) -> None:
     fid = _fn(f)
     if fid not in _FLASH_IDS:
         raise MadiError(-9, "kFlash", f"handle {fid} is not an encoder attention kernel")
-    call("madi_flash_enc_f16", ptr(out), ptr(q), ptr(k), ptr(v), seq, nh)
+    calls.madi_flash_enc_f16(out, q, k, v, seq, nh)
 
 
 _FLASH_IDS = None
@@ -251,72 +252,71 @@ _FLASH_IDS = None
 def matmulF16Batched(a, b, c, m: int, n: int, k: int, alpha: float = 1.0,
                      beta: float = 0.0) -> None:
     """metal_backend.zig:120 -> mtl_matmul_f16_enc (metal_backend.h:103)."""
-    call("madi_matmul_f16", ptr(a), ptr(b), ptr(c), m, n, k, alpha, beta)
+    calls.madi_matmul_f16(a, b, c, m, n, k, alpha, beta)
 
 
 # ---- decoder.zig -----------------------------------------------------------
 def kGemvQ8(out, x, w: Q8, n: int, k: int) -> None:
     """decoder.zig:155-160 (gemv_q8)."""
-    call("madi_q8_gemv", ptr(out), ptr(x), w.qs, w.scales, n, k)
+    calls.madi_q8_gemv(out, x, w.qs, w.scales, n, k)
 
 
 def kGemvQ8Bias(out, x, w: Q8, bias, n: int, k: int) -> None:
     """decoder.zig:162-167 (gemv_q8_bias)."""
-    call("madi_q8_gemv_bias", ptr(out), ptr(x), w.qs, w.scales, ptr(bias), n, k)
+    calls.madi_q8_gemv_bias(out, x, w.qs, w.scales, bias, n, k)
 
 
 def kGemvQ8BiasEpi(f, out, x, w: Q8, bias, n: int, k: int) -> None:
     """decoder.zig:176-181; f = the gemv_q8_bias_gelu or gemv_q8_bias_res handle
     (or its name)."""
-    call("madi_q8_gemv_epi", _fn(f), ptr(out), ptr(x), w.qs, w.scales, ptr(bias), n, k)
+    calls.madi_q8_gemv_epi(_fn(f), out, x, w.qs, w.scales, bias, n, k)
 
 
 def pproj(in_f32, w: Q8, out_f32, M: int, N: int, Kk: int) -> None:
     """decoder.zig:427-432 (pproj: kDeq + kCvt32 + matmulF16Batched + kCvt16)
     as one fused kernel.  in_f32 [M][Kk] -> out_f32 [M][N]."""
-    call("madi_q8_pproj", ptr(out_f32), ptr(in_f32), w.qs, w.scales, M, N, Kk)
+    calls.madi_q8_pproj(out_f32, in_f32, w.qs, w.scales, M, N, Kk)
 
 
 def proj(in16, in_f32, w16, out_f32, B: int, N: int, Kk: int) -> None:
     """decoder.zig:337-341 (proj: kCvt32 + matmulF16Batched + kCvt16 on the
     F16 copy w16 of a Q8 weight); in16 is the BScratch staging buffer.  A w16
     that deqW16 recorded runs the fused batched projection on the Q8 weight."""
-    call("madi_proj_f16w", ptr(out_f32), ptr(in_f32), ptr(w16), ptr(in16), B, N, Kk)
+    calls.madi_proj_f16w(out_f32, in_f32, w16, in16, B, N, Kk)
 
 
 def kQkv(q_out, x, w: Q8, qb, vb, kc, vc, pos, d: int = D) -> None:
     """decoder.zig:169-174 (gemv_q8_qkv); pos is a device u32."""
-    call("madi_q8_gemv_qkv", ptr(q_out), ptr(x), w.qs, w.scales, ptr(qb), ptr(vb), ptr(kc),
-         ptr(vc), ptr(pos), d)
+    calls.madi_q8_gemv_qkv(q_out, x, w.qs, w.scales, qb, vb, kc, vc, pos, d)
 
 
 # ---- transcribe.zig ----------------------------------------------------------
 def kLogitGemv(logits, qs: int, sc: int, x, vocab: int = VOCAB, dim: int = D) -> None:
     """transcribe.zig:4369-4374 (logit_gemv_q8)."""
-    call("madi_q8_logit_gemv", ptr(logits), qs, sc, ptr(x), vocab, dim)
+    calls.madi_q8_logit_gemv(logits, qs, sc, x, vocab, dim)
 
 
 def embLookup(out, qs: int, sc: int, tok, vocab: int = VOCAB, dim: int = D) -> None:
     """transcribe.zig:4361-4366 (gpu_emb_lookup_q8), tok a device u32."""
-    call("madi_q8_emb_lookup", ptr(out), qs, sc, ptr(tok), vocab, dim)
+    calls.madi_q8_emb_lookup(out, qs, sc, tok, vocab, dim)
 
 
 def embLookupIndirect(out, qs: int, sc: int, tokens, pos, vocab: int = VOCAB,
                       dim: int = D) -> None:
     """emb_lookup_indirect_q8 (graph_helpers.metal:354-367)."""
-    call("madi_q8_emb_lookup_indirect", ptr(out), qs, sc, ptr(tokens), ptr(pos), vocab, dim)
+    calls.madi_q8_emb_lookup_indirect(out, qs, sc, tokens, pos, vocab, dim)
 
 
 def prefillEmbed(out, qs: int, sc: int, tokens, pe, pos0: int, M: int, dim: int = D,
                  vocab: int = VOCAB) -> None:
     """decoder.zig:460-467 (emb_pe_rows_q8): out[m] = emb(tokens[m]) + pe[pos0 + m]
     over the tied Q8 tok_emb; tokens a device u32 [M], pe a device f32 table."""
-    call("madi_q8_emb_pe_rows", ptr(out), qs, sc, ptr(tokens), ptr(pe), dim, pos0, M, vocab)
+    calls.madi_q8_emb_pe_rows(out, qs, sc, tokens, pe, dim, pos0, M, vocab)
 
 
 def gemv_f16x(out, x16, w: Q8, n: int, k: int, bias=None, epilogue: int = EPI_NONE) -> None:
     """Q8 GEMV with fp16 activations (the measured decoder-GEMV configuration)."""
-    call("madi_q8_gemv_f16x", ptr(out), ptr(x16), w.qs, w.scales, ptr(bias), n, k, epilogue)
+    calls.madi_q8_gemv_f16x(out, x16, w.qs, w.scales, bias, n, k, epilogue)
 
 
 __all__ = [
