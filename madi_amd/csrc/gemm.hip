@@ -759,12 +759,14 @@ __device__ inline OutTile out_tile(const OutSeg &seg, void *C, const float *bias
   return {seg.c[s], seg.b[s], seg.n, p0 - s * (seg.n / kPanelRows), seg.n / kPanelRows};
 }
 
-template <int MT, int EPI, bool PADDED, bool F32 = false, bool TAIL = false, int PW = 2>
-__global__ __launch_bounds__(256) void q8_gemm_kernel(
+// SPLITS: K may be split over workgroups (the partials' registers and the
+// mapping's division are left out of the launches that never do).
+template <int MT, int EPI, bool PADDED, bool F32, bool TAIL, int PW, bool SPLITS>
+__device__ __forceinline__ void q8_gemm_body(
     const void *__restrict__ A, const uint8_t *__restrict__ qs, const f16 *__restrict__ sc,
     uint32_t M, uint32_t N, uint32_t K, uint32_t tiles_m, uint32_t tiles_n, uint32_t splits,
     uint32_t cper, uint32_t crem, void *__restrict__ Cout, const float *__restrict__ bias,
-    float *__restrict__ ws, uint32_t *__restrict__ cnt, const OutSeg seg) {
+    float *__restrict__ ws, uint32_t *__restrict__ cnt, const OutSeg &seg) {
   using G = Geometry<MT, F32, PW>;
   static_assert(!F32 || EPI == MADI_EPI_NONE, "f32 output has no bias epilogue");
   static_assert(!TAIL || (!PADDED && !F32 && MT >= 2 && PW == 2), "the m-tile-major tail's shapes");
@@ -794,7 +796,7 @@ __global__ __launch_bounds__(256) void q8_gemm_kernel(
   const uint32_t item = first + (L >> 3);
   // launches that never split K (the m-tile-major tail, the f16 128-column
   // tiles: the host checks) skip the division
-  constexpr bool kUnsplit = TAIL || (PW == 1 && !F32);
+  constexpr bool kUnsplit = TAIL || !SPLITS;
   const uint32_t bid = kUnsplit ? item : item / splits, split = kUnsplit ? 0u : item - bid * splits;
   const uint32_t tile = bid;
   const uint32_t group_m = tiles_m < 6 ? tiles_m : 6;
@@ -942,8 +944,7 @@ __global__ __launch_bounds__(256) void q8_gemm_kernel(
   wait_then_barrier<0>();
   // f16 launches of 128-column tiles run unsplit (the host checks), and leave
   // the reduction's registers out of their allocation
-  constexpr bool kSplits = PW == 2 || F32;
-  if constexpr (kSplits) {
+  if constexpr (SPLITS) {
   if (splits > 1) {
     // Split K: every workgroup of the tile publishes its partial sums (in
     // register order, so each lane later reads back exactly what it wrote) and
@@ -1139,6 +1140,30 @@ __global__ __launch_bounds__(256) void q8_gemm_kernel(
       if (n < ot.n) __builtin_amdgcn_raw_buffer_store_b128(v, cr, (row * ot.n + n) * 2, 0, kSc1);
     }
   }
+}
+
+template <int MT, int EPI, bool PADDED, bool F32 = false, bool TAIL = false, int PW = 2>
+__global__ __launch_bounds__(256) void q8_gemm_kernel(
+    const void *__restrict__ A, const uint8_t *__restrict__ qs, const f16 *__restrict__ sc,
+    uint32_t M, uint32_t N, uint32_t K, uint32_t tiles_m, uint32_t tiles_n, uint32_t splits,
+    uint32_t cper, uint32_t crem, void *__restrict__ Cout, const float *__restrict__ bias,
+    float *__restrict__ ws, uint32_t *__restrict__ cnt, const OutSeg seg) {
+  // f16 launches of 128-column tiles run unsplit (the host checks)
+  q8_gemm_body<MT, EPI, PADDED, F32, TAIL, PW, !TAIL && (PW == 2 || F32)>(
+      A, qs, sc, M, N, K, tiles_m, tiles_n, splits, cper, crem, Cout, bias, ws, cnt, seg);
+}
+
+// 64 x 128 tiles with K split over workgroups (madi_q8_gemm's long K with few
+// rows): an instance of its own, as the split's registers slow the unsplit
+// 128-column tiles.
+template <int EPI>
+__global__ __launch_bounds__(256) void q8_gemm_narrow_split_kernel(
+    const void *__restrict__ A, const uint8_t *__restrict__ qs, const f16 *__restrict__ sc,
+    uint32_t M, uint32_t N, uint32_t K, uint32_t tiles_m, uint32_t tiles_n, uint32_t splits,
+    uint32_t cper, uint32_t crem, void *__restrict__ Cout, const float *__restrict__ bias,
+    float *__restrict__ ws, uint32_t *__restrict__ cnt, const OutSeg seg) {
+  q8_gemm_body<2, EPI, false, false, false, 1, true>(A, qs, sc, M, N, K, tiles_m, tiles_n, splits,
+                                                     cper, crem, Cout, bias, ws, cnt, seg);
 }
 
 // ---------------------------------------------------------------- persistent tile loop
@@ -1857,10 +1882,16 @@ int launch_gemm(const void *A, const uint8_t *qs, const f16 *sc, void *C, const 
   };
   if constexpr (PW == 1) {
     // 128-column tiles: the host chooses them only for unpadded K loops, and
-    // for the f16 GEMM only unsplit
-    if (padded || (!F32 && splits != 1))
+    // for the f16 GEMM split only at 64 rows
+    if (padded || (!F32 && MT != 2 && splits != 1))
       return fail(MADI_ERR_SHAPE, "%s: 128-column tiles need an unpadded%s K loop",
-                  F32 ? "madi_q8_pproj" : "madi_q8_gemm", F32 ? "" : ", unsplit");
+                  F32 ? "madi_q8_pproj" : "madi_q8_gemm", F32 || MT == 2 ? "" : ", unsplit");
+    if constexpr (!F32 && MT == 2) {
+      if (splits != 1) {
+        go(q8_gemm_narrow_split_kernel<EPI>);
+        return check_launch("madi_q8_gemm");
+      }
+    }
     go(q8_gemm_kernel<MT, EPI, false, F32, false, 1>);
   } else if (padded)
     go(q8_gemm_kernel<MT, EPI, true, F32>);
@@ -1887,6 +1918,17 @@ int dispatch_epi(int epi, const f16 *A, const uint8_t *qs, const f16 *sc, f16 *C
     return launch_gemm<MT, MADI_EPI_BIAS_GELU, false, PW>(A, qs, sc, C, bias, M, N, K, where, seg);
   default: return fail(MADI_ERR_ARG, "madi_q8_gemm: unknown epilogue %d", epi);
   }
+}
+
+// Whether a long K on few rows runs 64 x 128 tiles split over workgroups
+// instead of 64 x 256 ones: where their split count leaves an unpadded K loop
+// and one round of workgroups.  Twice the workgroups at the same split count,
+// or half the splits (and partial sums) at the same workgroups (5120 -> 1280
+// + bias, 64 x 256 / 64 x 128, us: M = 128 15.6 / 10.9, 256 15.9 / 11.4, 320
+// 16.1 / 14.3, 384 17.2 / 13.8, 600 20.1 / 16.0, 768 20.6 / 17.6).
+bool narrow_split(uint32_t m, uint32_t n, uint32_t k) {
+  const uint32_t chunks = k / kChunkK, tiles = tile_count(m, n, 2, 1), splits = split_count(tiles, chunks);
+  return narrow_ok(k) && splits > 1 && tiles * splits <= (uint32_t)cu_count() && !loop_padded(chunks, splits);
 }
 
 int q8_gemm(const char *what, const void *a, const void *qs, const void *scales, void *c,
@@ -1935,6 +1977,7 @@ int q8_gemm(const char *what, const void *a, const void *qs, const void *scales,
       default: return fail(MADI_ERR_ARG, "%s: unknown epilogue %d", what, epilogue);
       }
     }
+    if (narrow_split(m, n, k)) return dispatch_epi<2, 1>(epilogue, A, Q, S, C, bias, m, n, k, where, seg);
     return dispatch_epi<kSplitTile>(epilogue, A, Q, S, C, bias, m, n, k, where, seg);
   }
   // Otherwise the lowest tiles whose count still fits one workgroup per CU:
