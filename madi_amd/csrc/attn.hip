@@ -18,8 +18,9 @@
 // projection GEMMs' output, unpadded: rows past seq are never read -- row
 // indices clamp to the last row, and the keys past seq get weight 0).
 //
-// Workgroup: 128 query rows of one head.  A key group of 4 waves walks a
-// range of the keys; wave w owns query rows 32w..32w+31 (the MFMA's 32
+// Workgroup: 128 query rows of one head (32 or 64 where those still give at
+// most one workgroup per CU; a key group then has one or two waves).  A key
+// group of 4 waves walks a range of the keys; wave w owns query rows 32w..32w+31 (the MFMA's 32
 // columns).  KS key groups (KS waves per SIMD) split the key range and merge
 // their partial (m', sum, O) in LDS at the end; the default is four, whose
 // waves overlap each other's matrix and vector work.  Per 64-key block a
@@ -93,22 +94,24 @@ __device__ inline void wait_q_then_barrier(u32x4 (&qf)[4]) {
                : "memory");
 }
 
-// Grid: one workgroup per (head, 128-row query tile), 256 * KS threads: KS
-// key groups of four waves.  PIPE: the next block's S during this block's
+// Grid: one workgroup per (head, query tile of 32 QW rows), 64 QW KS threads:
+// KS key groups of QW waves.  PIPE: the next block's S during this block's
 // softmax (two key groups, two waves per SIMD); otherwise S at the start of
 // each block and the three or four waves per SIMD overlap each other.
-template <int KS, bool PIPE>
-__global__ __launch_bounds__(256 * KS) void flash_enc_kernel(
-    f16 *__restrict__ out, const f16 *__restrict__ q, const f16 *__restrict__ k,
-    const f16 *__restrict__ v, uint32_t seq, uint32_t nh, uint32_t qtiles) {
+template <int KS, bool PIPE, int QW>
+__device__ __forceinline__ void flash_enc(f16 *__restrict__ out, const f16 *__restrict__ q,
+                                          const f16 *__restrict__ k, const f16 *__restrict__ v,
+                                          uint32_t seq, uint32_t nh, uint32_t qtiles) {
   constexpr int NS = kStages<KS, PIPE>;
   constexpr int RB = kRingBytes<KS, PIPE>;
   static_assert(KS * RB <= 160 * 1024, "LDS");
-  static_assert((KS - 1) * 4 * 34 * 64 * 4 <= KS * RB, "exchange area");
+  static_assert((KS - 1) * QW * 34 * 64 * 4 <= KS * RB, "exchange area");
+  static_assert(QW == 4 || NS == 2, "the waits below count four waves' DMAs");
+  constexpr int kCopy = 64 / QW, kDmas = kCopy / 8;  // rows and DMAs of a tile per wave
   __shared__ __attribute__((aligned(1024))) uint8_t smem[KS * RB];
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t wave = sgpr(threadIdx.x >> 6);
-  const uint32_t grp = wave >> 2, wq = wave & 3;
+  const uint32_t grp = wave / QW, wq = wave % QW;
   const uint32_t h = lane >> 5, r = lane & 31;
 
   // Workgroups x and x + 8 run on the same XCD (round-robin dispatch): each
@@ -124,7 +127,7 @@ __global__ __launch_bounds__(256 * KS) void flash_enc_kernel(
   const desc_t dq = make_desc(q, bytes), dk = make_desc(k, bytes), dv = make_desc(v, bytes);
 
   // Q^T fragments (B operand of S^T): query row q0 + r, d = 16s + 8h .. +7
-  const uint32_t q0 = qt * kQRows + wq * 32;
+  const uint32_t q0 = (qt * QW + wq) * 32;
   const uint32_t qrow = min(q0 + r, seq - 1);
   u32x4 qf[4];
   {
@@ -144,29 +147,29 @@ __global__ __launch_bounds__(256 * KS) void flash_enc_kernel(
   const uint32_t iters = (nb + KS - 1) / KS;
   const uint32_t ring = lds_addr(smem) + grp * RB;
 
-  // DMA plan: wave wq copies rows 16wq .. 16wq+15 of the K and V tiles, 8 rows
-  // per DMA; lane -> row 16wq + 8i + lane/8, LDS piece lane%8, which holds the
-  // row's logical piece (lane%8) ^ swizzle(row)
-  uint32_t k_dma[2], v_dma[2], drow[2];
+  // DMA plan: wave wq copies kCopy rows of the K and V tiles from kCopy wq on,
+  // 8 rows per DMA; lane -> row kCopy wq + 8i + lane/8, LDS piece lane%8,
+  // which holds the row's logical piece (lane%8) ^ swizzle(row)
+  uint32_t k_dma[kDmas], v_dma[kDmas], drow[kDmas];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    drow[i] = 16 * wq + 8 * i + (lane >> 3);
+  for (int i = 0; i < kDmas; ++i) {
+    drow[i] = kCopy * wq + 8 * i + (lane >> 3);
     k_dma[i] = head * 128 + 16 * ((lane & 7) ^ swz_k(drow[i]));
     v_dma[i] = head * 128 + 16 * ((lane & 7) ^ swz_v(drow[i]));
   }
   auto issue = [&](uint32_t blk, uint32_t stage) {
     const uint32_t kv0 = (kb0 + blk) * 64;
-    const uint32_t kt = ring + stage * kStageBytes + 16 * wq * 128;
+    const uint32_t kt = ring + stage * kStageBytes + kCopy * wq * 128;
     if (kv0 + 64 <= seq) {  // a whole block: the block offset is a scalar
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < kDmas; ++i) {
         const uint32_t row = drow[i] * rowb;
         dma16<0, true>(dk, row + k_dma[i], kv0 * rowb, kt + i * 1024);
         dma16<0, true>(dv, row + v_dma[i], kv0 * rowb, kt + kTileBytes + i * 1024);
       }
     } else {  // the last block: rows past seq repeat the last row
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < kDmas; ++i) {
         const uint32_t row = min(kv0 + drow[i], seq - 1) * rowb;
         dma16<0, true>(dk, row + k_dma[i], 0, kt + i * 1024);
         dma16<0, true>(dv, row + v_dma[i], 0, kt + kTileBytes + i * 1024);
@@ -411,7 +414,7 @@ __global__ __launch_bounds__(256 * KS) void flash_enc_kernel(
     // ring is free: every wave passed the loop's last barrier); a group
     // without blocks hands m' = -inf, sum 0, O 0, which weigh nothing
     float *base = reinterpret_cast<float *>(smem) + wq * 34 * 64;
-    constexpr int kSlot = 4 * 34 * 64;  // floats per key group
+    constexpr int kSlot = QW * 34 * 64;  // floats per key group
     if (grp > 0) {
       float *xch = base + (grp - 1) * kSlot;
       xch[lane] = mref;
@@ -460,6 +463,20 @@ __global__ __launch_bounds__(256 * KS) void flash_enc_kernel(
   }
 }
 
+template <int KS, bool PIPE>
+__global__ __launch_bounds__(256 * KS) void flash_enc_kernel(
+    f16 *__restrict__ out, const f16 *__restrict__ q, const f16 *__restrict__ k,
+    const f16 *__restrict__ v, uint32_t seq, uint32_t nh, uint32_t qtiles) {
+  flash_enc<KS, PIPE, 4>(out, q, k, v, seq, nh, qtiles);
+}
+// Short sequences: tiles of 32 or 64 query rows.
+template <int QW>
+__global__ __launch_bounds__(256 * QW) void flash_short_kernel(
+    f16 *__restrict__ out, const f16 *__restrict__ q, const f16 *__restrict__ k,
+    const f16 *__restrict__ v, uint32_t seq, uint32_t nh, uint32_t qtiles) {
+  flash_enc<4, false, QW>(out, q, k, v, seq, nh, qtiles);
+}
+
 bool overlaps(const void *a, size_t an, const void *b, size_t bn) {
   const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
   return x < y + bn && y < x + an;
@@ -484,6 +501,14 @@ void launch_flash(void *out, const void *q, const void *k, const void *v, uint32
       (f16 *)out, (const f16 *)q, (const f16 *)k, (const f16 *)v, seq, nh, qtiles);
 }
 
+template <int QW>
+int launch_short(void *out, const void *q, const void *k, const void *v, uint32_t seq, uint32_t nh) {
+  const uint32_t qtiles = (seq + 32 * QW - 1) / (32 * QW);
+  flash_short_kernel<QW><<<nh * qtiles, 256 * QW, 0, stream()>>>(
+      (f16 *)out, (const f16 *)q, (const f16 *)k, (const f16 *)v, seq, nh, qtiles);
+  return check_launch("madi_flash_enc_f16");
+}
+
 }  // namespace
 
 extern "C" int madi_flash_enc_f16(void *out, const void *q, const void *k, const void *v,
@@ -504,6 +529,17 @@ extern "C" int madi_flash_enc_f16(void *out, const void *q, const void *k, const
     if (int rc = deferred_before_read(in, bytes)) return rc;
   if (int rc = deferred_before_write(out, bytes)) return rc;
   const uint32_t qtiles = (seq_len + kQRows - 1) / kQRows;
+  if (key_groups() == 4) {
+    // The smallest query tile that leaves one workgroup per CU: fewer waves
+    // share a SIMD, and a tile's K loop, merge and stores shrink with it (20
+    // heads, 128- / 64- / 32-row tiles, us: 100 frames 6.7 / 5.5 / 4.9, 375 9.4
+    // / 7.1 / 6.4, 750 12.2 / 8.9 / -; 6 heads: 1250 15.8 / 11.1 / 10.4, 2000
+    // 21.4 / 15.2 / -).  A second round costs more than that saves (20 heads,
+    // 400 frames: 32-row 11.3, 64-row 7.2; 800: 64-row 17.5, 128-row 12.9).
+    const uint64_t cus = (uint64_t)cu_count(), t32 = (seq_len + 31) / 32, t64 = (seq_len + 63) / 64;
+    if (t32 * nh <= cus) return launch_short<1>(out, q, k, v, seq_len, nh);
+    if (t64 * nh <= cus) return launch_short<2>(out, q, k, v, seq_len, nh);
+  }
   switch (key_groups()) {
   case 1: launch_flash<1, true>(out, q, k, v, seq_len, nh, qtiles); break;
   case 2: launch_flash<2, true>(out, q, k, v, seq_len, nh, qtiles); break;
