@@ -82,8 +82,13 @@ __device__ inline uint32_t swz_b(uint32_t row) { return (row & 3) << 2; }
 
 // Grid: one workgroup per tile, the grid rounded up to a multiple of 8.
 // Workgroups x and x + 8 run on the same XCD (round-robin dispatch), so each
-// XCD takes a contiguous run of tiles, column tiles outermost, and the B
-// columns of a run are fetched into one L2.  M rows past the last are read
+// XCD takes a contiguous run of tiles, walked in groups of group_m row tiles
+// with column tiles outermost, and the operands of a run are fetched into one
+// L2.  Up to 12 row tiles are one group; more go in sixes, so that a run is
+// nearly square: 30 tiles of 64 x 128 over all 24 row tiles of 1500 rows read
+// the whole of A into every L2 (5120 -> 1280 30.8 -> 27.9 us, 1280 -> 1280 + bias
+// 9.8 -> 9.2, 1000 rows of 5120 -> 1280 27.3 -> 24.4; groups of 3, 4, 8 28.6,
+// 29.2, 28.8).  M rows past the last are read
 // as the last row (in bounds) and never stored.  Requires K % 64 == 0,
 // N % BN == 0, A, B, C and bias 16-byte aligned.  F32O: C is f32 (the
 // unrounded sums, no epilogue) instead of f16.
@@ -99,7 +104,8 @@ __device__ inline uint32_t swz_b(uint32_t row) { return (row & 3) << 2; }
 template <class G, int EPI, bool F32O>
 __global__ __launch_bounds__(512) void f16_nn_gemm_kernel(
     const f16 *__restrict__ A, const f16 *__restrict__ B, uint32_t M, uint32_t N, uint32_t K,
-    uint32_t tiles_m, uint32_t tiles, void *__restrict__ C, const float *__restrict__ bias) {
+    uint32_t tiles_m, uint32_t tiles_n, uint32_t tiles, uint32_t group_m, void *__restrict__ C,
+    const float *__restrict__ bias) {
   constexpr int S = G::kStages, BN = G::BN, TMw = G::kTM, TNw = G::kTN, WNw = G::kWN;
   static_assert(!F32O || EPI == MADI_EPI_NONE, "the f32 result takes no epilogue");
   constexpr uint32_t kOut = F32O ? 4 : 2;  // bytes per C element
@@ -113,7 +119,14 @@ __global__ __launch_bounds__(512) void f16_nn_gemm_kernel(
   const uint32_t slot = b >> 3;
   if (slot >= per + (x < extra ? 1u : 0u)) return;
   const uint32_t item = x * per + (x < extra ? x : extra) + slot;
-  const uint32_t tn = item / tiles_m, tm = item - tn * tiles_m;
+  uint32_t first_m = 0, in = item, gm = tiles_m;
+  if (group_m < tiles_m) {
+    const uint32_t per_group = group_m * tiles_n, gi = item / per_group;
+    first_m = gi * group_m;
+    in = item - gi * per_group;
+    gm = tiles_m - first_m < group_m ? tiles_m - first_m : group_m;
+  }
+  const uint32_t tn = in / gm, tm = first_m + (in - tn * gm);
   const uint32_t m0 = tm * G::BM, n0 = tn * BN, nk = K / 64;
   const uint32_t ring = lds_addr(smem);
   constexpr uint32_t kPieces = BN * kOut / 16;  // 16-byte pieces per tile row
@@ -364,9 +377,10 @@ template <class G, int EPI, bool F32O = false>
 int launch_nn(const void *a, const void *b, void *c, const float *bias, uint32_t m, uint32_t n,
               uint32_t k, const char *what) {
   const uint32_t tiles_m = (m + G::BM - 1) / G::BM, tiles = tiles_m * (n / G::BN);
+  const uint32_t group_m = tiles_m > 12 ? 6 : tiles_m;
   hipLaunchKernelGGL((f16_nn_gemm_kernel<G, EPI, F32O>), dim3((tiles + 7) & ~7u), dim3(512), 0,
                      stream(), static_cast<const f16 *>(a), static_cast<const f16 *>(b), m, n, k,
-                     tiles_m, tiles, c, bias);
+                     tiles_m, n / G::BN, tiles, group_m, c, bias);
   return check_launch(what);
 }
 
