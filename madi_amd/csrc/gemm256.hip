@@ -6,7 +6,7 @@
 // pipes 66 % busy, so what pays is less energy per product.  Three things do
 // that here.  The panel-layout weight is written once per call as F16 [N][K]
 // rows into the library's scratch (the exact fp16_rne(q * s) of every other
-// kernel, 4 us for 5120 x 1280) instead of being dequantised once per 128-row
+// kernel, 6.4 us for 5120 x 1280) instead of being dequantised once per 128-row
 // tile beside the MFMAs.  The MFMA is 16x16x32: a register-only loop on random
 // operands sustains 1.91 PFLOP/s with it and 1.58-1.68 with 32x32x16 (both
 // 2.4 on zeros), because each product updates half as many accumulators.  And
