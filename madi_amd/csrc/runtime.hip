@@ -139,7 +139,7 @@ extern "C" int madi_init(void) {
                 prop.gcnArchName);
   g_cu_count = prop.multiProcessorCount;
   g_init = true;
-  // A workspace big enough for every split GEMV / projection (and small
+  // A workspace big enough for every split projection (and small
   // split GEMMs) from the start, so those never allocate later (e.g. while a
   // caller captures a graph).
   float *partials = nullptr;
