@@ -1831,13 +1831,17 @@ bool use_tail(uint32_t splits, uint32_t chunks) {
 enum Scratch { kWorkspace = 0, kStatic = 1 };
 
 // Scratch for a weight dequantised by the call (gemm256.hip), from where the
-// call's split-K partials would come; nullptr if there is not enough.
+// call's split-K partials would come; nullptr if there is not enough.  Nor
+// during a graph capture: a replay is not ordered with the library's other
+// calls, and the kernels that run instead share no memory with them.
 void *weight_scratch(size_t bytes, Scratch where) {
   if (where == kStatic) {
     uint8_t *base = nullptr;
     if (resolve_scratch(&base) != MADI_OK) return nullptr;
     return base + kScratchCounters * 4;
   }
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream(), &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return nullptr;
   float *ws = nullptr;
   uint32_t *cnt = nullptr;
   return workspace_try(bytes, &ws, &cnt) ? ws : nullptr;
@@ -2008,8 +2012,8 @@ int q8_gemm(const char *what, const void *a, const void *qs, const void *scales,
   if (seg.n) return kSegUnsupported;
   // many rows: 256 x 256 tiles on the weight dequantised once into scratch,
   // where the fixed array holds it too (so that both entry points take the
-  // same kernel).  A workspace that would have to grow during a graph capture
-  // leaves the call to the kernels below.
+  // same kernel).  Without the workspace (a graph capture, no memory) the
+  // kernels below take the call.
   if (gemm256_suits(m, n, k, kScratchBytes - kScratchCounters * 4))
     if (void *w16 = weight_scratch(gemm256_bytes(n, k), where))
       return gemm256(A, Q, S, C, bias, m, n, k, epilogue, w16);
