@@ -149,10 +149,11 @@ int madi_q8_gemm(const void *a, const void *qs, const void *scales, void *c,
 /* No counterpart in the reference: madi_q8_gemm for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Same arguments, kernels and results as
- * madi_q8_gemm, bit for bit (many rows outside a graph capture: within one,
- * madi_q8_gemm sums them in another order); where a shape splits K over workgroups, the
- * partial sums and arrival counters, and where many rows run on a weight
- * dequantised once, that weight, live in a fixed 16 MiB device array of
+ * madi_q8_gemm, bit for bit (both outside a graph capture or both within one:
+ * a captured call sums many rows in another order than an eager one); where a
+ * shape splits K over workgroups, the partial sums and arrival counters, and
+ * where many rows run on a weight dequantised once, that weight, live in a
+ * fixed 16 MiB device array of
  * the library (MADI_Q8_GEMM_NOALLOC_SCRATCH bytes per GPU, held until the
  * process ends) instead of the growable workspace, so the call allocates
  * nothing.  Every split shape of madi_q8_gemm fits (at most 15 MiB of

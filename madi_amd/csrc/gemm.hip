@@ -1830,18 +1830,28 @@ bool use_tail(uint32_t splits, uint32_t chunks) {
 // Where a launch keeps its split-K partials and counters.
 enum Scratch { kWorkspace = 0, kStatic = 1 };
 
+// Whether the stream is being captured.  A query that fails (the legacy null
+// stream while another stream captures) counts as a capture, and its error is
+// not the launch's that follows.
+bool capturing() {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream(), &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
 // Scratch for a weight dequantised by the call (gemm256.hip), from where the
 // call's split-K partials would come; nullptr if there is not enough.  Nor
-// during a graph capture: a replay is not ordered with the library's other
-// calls, and the kernels that run instead share no memory with them.
+// during a graph capture, at either entry point: a replay is not ordered with
+// the library's other calls, and the kernels that run instead share no memory
+// with them.
 void *weight_scratch(size_t bytes, Scratch where) {
+  if (capturing()) return nullptr;
   if (where == kStatic) {
     uint8_t *base = nullptr;
     if (resolve_scratch(&base) != MADI_OK) return nullptr;
     return base + kScratchCounters * 4;
   }
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream(), &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return nullptr;
   float *ws = nullptr;
   uint32_t *cnt = nullptr;
   return workspace_try(bytes, &ws, &cnt) ? ws : nullptr;

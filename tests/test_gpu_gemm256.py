@@ -66,6 +66,54 @@ def test_tiles_against_oracle(q, m, n, k, epi):
         assert np.array_equal(big.cpu().numpy(), out), name
 
 
+def capture(q, call):
+    """A graph of `call`, captured on a stream of its own."""
+    torch.cuda.synchronize()
+    g, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(g, stream=side):
+            q.init(side)
+            call()
+    q.init()
+    return g
+
+
+def test_captured_noalloc_is_the_captured_gemm(q):
+    """Captured, the two entry points take the same kernels (the fused ones,
+    which share no memory with other calls): the same bits, over replays with
+    eager calls of another weight through the fixed scratch between them."""
+    m, n, k = 6000, 5120, 1280
+    say(f"gemm256 noalloc capture m={m} n={n} k={k}")
+    a, qs, sc = synth.gemm_case(11, m, n, k)
+    bias = np.random.default_rng(12).standard_normal(n).astype(np.float32)
+    w, a_d, b_d = q.upload_q8(qs, sc), dev_f16(a), dev(bias)
+    a2, qs2, sc2 = synth.gemm_case(13, m, n, k)
+    w2, a2_d = q.upload_q8(qs2, sc2), dev_f16(a2)
+    outs, graphs = [], []
+    for name in ("madi_q8_gemm", "madi_q8_gemm_noalloc"):
+        c = torch.empty((m, n), dtype=torch.int16, device="cuda")
+        args = (a_d.data_ptr(), w.qs, w.scales, c.data_ptr(), b_d.data_ptr(), m, n, k, O.EPI_BIAS)
+        graphs.append(capture(q, lambda: _lib.call(name, *args)))
+        outs.append(c)
+    eager = torch.empty((m, n), dtype=torch.int16, device="cuda")
+    first = None
+    for rep in range(3):
+        for g, c in zip(graphs, outs):
+            c.fill_(-1)
+            g.replay()
+            torch.cuda.synchronize()
+            if first is None:
+                first = c.cpu().numpy()
+                rows = np.unique(np.r_[0, 127, 128, 255, 256, 3000, m - 1])
+                check(host_f16(c), a, qs, sc, bias, O.EPI_BIAS, rows)
+            assert np.array_equal(c.cpu().numpy(), first), rep
+            _lib.call("madi_q8_gemm_noalloc", a2_d.data_ptr(), w2.qs, w2.scales, eager.data_ptr(),
+                      b_d.data_ptr(), m, n, k, O.EPI_BIAS)
+            q.sync()
+    check(host_f16(eager), a2, qs2, sc2, bias, O.EPI_BIAS, rows)
+
+
 def test_captured_calls_share_no_scratch(q):
     """A captured call runs the fused kernels, whether the workspace (4 MiB
     after madi_init, smaller than the 13 MB weight of 6000 x 1280 -> 5120) has
