@@ -142,24 +142,27 @@ int madi_q8_dequant_f16(void *wdq, const void *qs, const void *scales, uint32_t 
  * replaces the encoder's kDeq + kM4 / kM4Bias pairs (encoder.zig:125-136,
  * 262-301) and mul_mm_q8 (q8_gemm.metal:29-102).  epilogue: NONE, BIAS or
  * BIAS_GELU (bias may be NULL for NONE).  Requires N % 32 == 0, K % 64 == 0,
- * 16-byte aligned A and C. */
+ * 16-byte aligned A and C.  Many rows (a long recording's) of a weight below
+ * 8 Mi elements run on that weight dequantised once per call into a second
+ * fixed 16 MiB array of the library; within a graph capture they do not (a
+ * replay may overlap other calls), and a captured call then sums in another
+ * order than an eager one: both are within fp32 accumulation, not the same
+ * bits. */
 int madi_q8_gemm(const void *a, const void *qs, const void *scales, void *c,
                  const float *bias, uint32_t m, uint32_t n, uint32_t k, int epilogue);
 
 /* No counterpart in the reference: madi_q8_gemm for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Same arguments, kernels and results as
- * madi_q8_gemm, bit for bit (both outside a graph capture or both within one:
- * a captured call sums many rows in another order than an eager one); where a
- * shape splits K over workgroups, the partial sums and arrival counters, and
- * where many rows run on a weight dequantised once, that weight, live in a
- * fixed 16 MiB device array of
- * the library (MADI_Q8_GEMM_NOALLOC_SCRATCH bytes per GPU, held until the
- * process ends) instead of the growable workspace, so the call allocates
- * nothing.  Every split shape of madi_q8_gemm fits (at most 15 MiB of
- * partials); a larger need fails with MADI_ERR_SHAPE.  All calls on one GPU
- * share that GPU's array: calls that overlap on one GPU (several streams or
- * host threads) race and must not. */
+ * madi_q8_gemm, bit for bit (both eager or both captured, see there); where a
+ * shape splits K over workgroups, the partial sums and arrival counters live
+ * in a fixed 16 MiB device array of the library
+ * (MADI_Q8_GEMM_NOALLOC_SCRATCH bytes per GPU, held until the process ends)
+ * instead of the growable workspace, so the call allocates nothing.  Every
+ * split shape of madi_q8_gemm fits (at most 15 MiB of partials); a larger
+ * need fails with MADI_ERR_SHAPE.  All calls on one GPU share that GPU's
+ * array: calls that overlap on one GPU (several streams or host threads) race
+ * and must not. */
 #define MADI_Q8_GEMM_NOALLOC_SCRATCH (16u << 20)
 int madi_q8_gemm_noalloc(const void *a, const void *qs, const void *scales, void *c,
                          const float *bias, uint32_t m, uint32_t n, uint32_t k, int epilogue);

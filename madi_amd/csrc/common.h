@@ -25,9 +25,6 @@ int cu_count();
 // The counters come first, kWorkspaceCounterBytes of them, then the partials.
 constexpr size_t kWorkspaceCounterBytes = 16384 * 4;
 int workspace(size_t partial_bytes, size_t counters, float **partials, uint32_t **cnt);
-// The same for a caller that has another way: false, with no error recorded,
-// where the workspace cannot grow (a graph capture, no memory).
-bool workspace_try(size_t partial_bytes, float **partials, uint32_t **cnt);
 // Releases the fp16 GEMM's rocBLAS handle (madi_cleanup).
 void f16gemm_cleanup();
 // The MFMA GEMM with f32 activations (rounded to f16) and an f32 result, for
@@ -57,8 +54,9 @@ struct OutSeg {
 constexpr int kSegUnsupported = 1;
 int q8_gemm_seg(const void *a, const void *qs, const void *scales, const OutSeg &seg, uint32_t m,
                 uint32_t n, uint32_t k, int epilogue);
-// Resolves the current device's address of the allocation-free GEMM's fixed
-// scratch array and clears its counters (madi_init).
+// Resolves the current device's addresses of the library's fixed arrays (the
+// allocation-free GEMM's scratch, whose counters it clears, and the many-row
+// GEMM's weight; madi_init).
 int gemm_scratch_init();
 
 // Deferred dequantisation (boundary.hip).  madi_q8_dequant_f16 records

@@ -1840,23 +1840,6 @@ bool capturing() {
   return true;
 }
 
-// Scratch for a weight dequantised by the call (gemm256.hip), from where the
-// call's split-K partials would come; nullptr if there is not enough.  Nor
-// during a graph capture, at either entry point: a replay is not ordered with
-// the library's other calls, and the kernels that run instead share no memory
-// with them.
-void *weight_scratch(size_t bytes, Scratch where) {
-  if (capturing()) return nullptr;
-  if (where == kStatic) {
-    uint8_t *base = nullptr;
-    if (resolve_scratch(&base) != MADI_OK) return nullptr;
-    return base + kScratchCounters * 4;
-  }
-  float *ws = nullptr;
-  uint32_t *cnt = nullptr;
-  return workspace_try(bytes, &ws, &cnt) ? ws : nullptr;
-}
-
 template <int MT, int EPI, bool F32 = false, int PW = 2>
 int launch_gemm(const void *A, const uint8_t *qs, const f16 *sc, void *C, const float *bias,
                 uint32_t M, uint32_t N, uint32_t K, Scratch where, const OutSeg &seg = OutSeg{}) {
@@ -2020,13 +2003,11 @@ int q8_gemm(const char *what, const void *a, const void *qs, const void *scales,
   if (tile_count(m, n, 3) <= cus)
     return dispatch_epi<3>(epilogue, A, Q, S, C, bias, m, n, k, where, seg);
   if (seg.n) return kSegUnsupported;
-  // many rows: 256 x 256 tiles on the weight dequantised once into scratch,
-  // where the fixed array holds it too (so that both entry points take the
-  // same kernel).  Without the workspace (a graph capture, no memory) the
-  // kernels below take the call.
-  if (gemm256_suits(m, n, k, kScratchBytes - kScratchCounters * 4))
-    if (void *w16 = weight_scratch(gemm256_bytes(n, k), where))
-      return gemm256(A, Q, S, C, bias, m, n, k, epilogue, w16);
+  // many rows: 256 x 256 tiles on the weight dequantised once.  Not within a
+  // graph capture: a replay is not ordered with the library's other calls,
+  // which write the same array; the kernels below share no memory.
+  if (gemm256_suits(m, n, k) && !capturing())
+    if (f16 *w16 = gemm256_weight()) return gemm256(A, Q, S, C, bias, m, n, k, epilogue, w16);
   // at least two rounds of 128-row tiles: the persistent tile loop
   if (persist_ok(m, n, k)) {
     switch (epilogue) {
@@ -2042,8 +2023,9 @@ int q8_gemm(const char *what, const void *a, const void *qs, const void *scales,
 }  // namespace
 
 namespace madi {
-// madi_init: the current device's scratch address, resolved at set-up.
+// madi_init: the current device's scratch addresses, resolved at set-up.
 int gemm_scratch_init() {
+  (void)gemm256_weight();
   uint8_t *base = nullptr;
   return resolve_scratch(&base);
 }

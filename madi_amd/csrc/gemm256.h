@@ -5,13 +5,16 @@
 
 namespace madi {
 
-// Whether the shape takes the 256 x 256 tiles, with at most max_scratch bytes
-// of scratch memory (16-byte aligned) for its dequantised weight, and how
-// many it needs.
-bool gemm256_suits(uint32_t m, uint32_t n, uint32_t k, size_t max_scratch);
-size_t gemm256_bytes(uint32_t n, uint32_t k);
+// Whether the shape takes the 256 x 256 tiles.
+bool gemm256_suits(uint32_t m, uint32_t n, uint32_t k);
+// The array that holds the dequantised weight during a call, on the current
+// device; nullptr if its address is not to be had.  It holds nothing else: the
+// split-K partials of a captured call, replayed on a stream of its own, must
+// not meet an eager call's weight.  Calls that use it are ordered by the
+// library's one stream.
+f16 *gemm256_weight();
 // Operands checked by madi_q8_gemm.
 int gemm256(const void *a, const uint8_t *qs, const f16 *sc, void *c, const float *bias, uint32_t m,
-            uint32_t n, uint32_t k, int epilogue, void *w16);
+            uint32_t n, uint32_t k, int epilogue, f16 *w);
 
 }  // namespace madi

@@ -5,7 +5,7 @@
 // long recording the fused kernels of gemm.hip run at 1.5 GHz with the matrix
 // pipes 66 % busy, so what pays is less energy per product.  Three things do
 // that here.  The panel-layout weight is written once per call as F16 [N][K]
-// rows into the library's scratch (the exact fp16_rne(q * s) of every other
+// rows into an array of the library (the exact fp16_rne(q * s) of every other
 // kernel, 6.4 us for 5120 x 1280) instead of being dequantised once per 128-row
 // tile beside the MFMAs.  The MFMA is 16x16x32: a register-only loop on random
 // operands sustains 1.91 PFLOP/s with it and 1.58-1.68 with 32x32x16 (both
@@ -311,29 +311,46 @@ int launch(const void *a, const f16 *w, void *c, const float *bias, uint32_t m, 
                      static_cast<const f16 *>(a), w, m, n, k, walk, static_cast<f16 *>(c), bias);
   return check_launch("madi_q8_gemm");
 }
+
+// The dequantised weight of the call in progress, one array per device.
+constexpr size_t kWeightBytes = size_t(16) << 20;
+static __device__ __align__(256) uint8_t weight_rows[kWeightBytes];
+constexpr int kMaxDevices = 64;
+f16 *g_weight[kMaxDevices];
 }  // namespace
 
-size_t gemm256_bytes(uint32_t n, uint32_t k) { return (size_t)n * k * 2; }
+f16 *gemm256_weight() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
+  if (!g_weight[dev]) {
+    void *ptr = nullptr;
+    if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(weight_rows)) != hipSuccess) {
+      (void)hipGetLastError();  // the launch that follows takes another kernel
+      return nullptr;
+    }
+    g_weight[dev] = static_cast<f16 *>(ptr);
+  }
+  return g_weight[dev];
+}
 
-// Whole 256-column groups (and byte offsets inside 2 GiB) whose tiles fill
-// their rounds of one tile per CU to at least nine tenths: a tile costs 0.87
-// to 0.9 of the two 128 x 256 tiles of the fused kernels (at M = 24000 1280 ->
+// Whole 256-column groups (a weight that fits its array, byte offsets inside
+// 2 GiB) whose tiles fill their rounds of one tile per CU to at least nine
+// tenths: a tile costs 0.87 to 0.9 of the two 128 x 256 tiles of the fused kernels (at M = 24000 1280 ->
 // 5120 + bias + GELU 351-366 -> 331-345 us, 5120 -> 1280 291-315 -> 268-283;
 // at M = 6000 1280 -> 5120 + GELU 95 -> 93), and a round that is emptier than
 // that gives it back (M = 5000, 400 tiles in two rounds, 91 -> 93 us; M =
 // 4000, 320 tiles, 71 -> 82).
-bool gemm256_suits(uint32_t m, uint32_t n, uint32_t k, size_t max_scratch) {
+bool gemm256_suits(uint32_t m, uint32_t n, uint32_t k) {
   const uint64_t cus = (uint64_t)cu_count() / 8 * 8;
-  if (n % kBN || cus == 0 || gemm256_bytes(n, k) > max_scratch || (uint64_t)n * 512 >= (1ull << 31))
+  if (n % kBN || cus == 0 || (uint64_t)n * k * 2 >= kWeightBytes || (uint64_t)n * 512 >= (1ull << 31))
     return false;
   const uint64_t tiles = (uint64_t)((m + kBM - 1) / kBM) * (n / kBN), rounds = (tiles + cus - 1) / cus;
   return tiles * 10 >= rounds * cus * 9;
 }
 
 int gemm256(const void *a, const uint8_t *qs, const f16 *sc, void *c, const float *bias, uint32_t m,
-            uint32_t n, uint32_t k, int epilogue, void *w16) {
+            uint32_t n, uint32_t k, int epilogue, f16 *w) {
   const uint32_t units = n / kPanelRows * (k / kChunkK);
-  f16 *w = static_cast<f16 *>(w16);
   hipLaunchKernelGGL(q8_rows_f16_kernel, dim3((units + 3) / 4), dim3(256), 0, stream(), w, qs, sc, k,
                      units);
   if (int rc = check_launch("madi_q8_gemm(rows)")) return rc;

@@ -84,13 +84,6 @@ int workspace(size_t partial_bytes, size_t counters, float **partials, uint32_t 
   return MADI_OK;
 }
 
-bool workspace_try(size_t partial_bytes, float **partials, uint32_t **cnt) {
-  if (workspace(partial_bytes, 0, partials, cnt) == MADI_OK) return true;
-  g_err[0] = 0;
-  (void)hipGetLastError();  // an allocation that failed is not the launch's error
-  return false;
-}
-
 int fail(int code, const char *fmt, ...) {
   va_list ap;
   va_start(ap, fmt);

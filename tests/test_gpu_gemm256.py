@@ -115,11 +115,9 @@ def test_captured_noalloc_is_the_captured_gemm(q):
 
 
 def test_captured_calls_share_no_scratch(q):
-    """A captured call runs the fused kernels, whether the workspace (4 MiB
-    after madi_init, smaller than the 13 MB weight of 6000 x 1280 -> 5120) has
-    grown since or not: the graphs' replays, with eager calls of the same
-    shape and another weight between, repeat their bits and are within the
-    bounds."""
+    """A captured call runs the fused kernels, before and after the first
+    eager one: the graphs' replays, with eager calls of the same shape and
+    another weight between, repeat their bits and are within the bounds."""
     m, n, k = 6000, 5120, 1280
     say(f"gemm256 capture m={m} n={n} k={k}")
     _lib.lib().madi_cleanup()
@@ -162,3 +160,65 @@ def test_captured_calls_share_no_scratch(q):
             q.sync()
     assert np.array_equal(first[0].view(np.uint16), first[1].view(np.uint16))
     check(host_f16(eager), a2, qs2, sc2, bias, O.EPI_BIAS_GELU, rows)
+
+
+def test_weight_is_not_in_the_workspace(q):
+    """An eager many-row call keeps its 13 MB weight out of the split-K
+    workspace (4 MiB after madi_init), which captured calls use: it takes no
+    device memory."""
+    m, n, k = 6000, 5120, 1280
+    _lib.lib().madi_cleanup()
+    q.init()
+    a, qs, sc = synth.gemm_case(5, m, n, k)
+    w, a_d = q.upload_q8(qs, sc), dev_f16(a)
+    c = torch.empty((m, n), dtype=torch.int16, device="cuda")
+    for call in (q.kGemmQ8, lambda *v: _lib.call("madi_q8_gemm_noalloc", v[0].data_ptr(), w.qs, w.scales,
+                                                 c.data_ptr(), None, m, n, k, O.EPI_NONE)):
+        q.sync()
+        before = torch.cuda.mem_get_info()[0]
+        call(a_d, w, c, m, n, k)
+        q.sync()
+        assert torch.cuda.mem_get_info()[0] == before
+
+
+def test_replayed_split_k_beside_an_eager_call(q):
+    """Split-K calls, captured, replay on a stream of their own while eager
+    many-row calls run on the library's: each result keeps its bits."""
+    say("gemm256 beside a replayed split K")
+    m, n, k = 6000, 5120, 1280
+    a, qs, sc = synth.gemm_case(21, m, n, k)
+    w, a_d = q.upload_q8(qs, sc), dev_f16(a)
+    ms, ns, ks = 300, 1280, 5120
+    a_s, qs_s, sc_s = synth.gemm_case(22, ms, ns, ks)
+    w_s, as_d = q.upload_q8(qs_s, sc_s), dev_f16(a_s)
+    x_d = dev(synth.activations(np.random.default_rng(23), 16, ks).astype(np.float32))
+
+    def new():
+        return (torch.empty((m, n), dtype=torch.int16, device="cuda"),
+                torch.empty((ms, ns), dtype=torch.int16, device="cuda"),
+                torch.empty((16, ns), dtype=torch.float32, device="cuda"))
+
+    def many(c):
+        q.kGemmQ8(a_d, w, c, m, n, k)
+
+    def split(c, p):
+        q.kGemmQ8(as_d, w_s, c, ms, ns, ks)
+        q.pproj(x_d, w_s, p, 16, ns, ks)
+
+    want, got = new(), new()
+    many(want[0])
+    split(*want[1:])
+    q.sync()
+    g, side = capture(q, lambda: split(*got[1:])), torch.cuda.Stream()
+    for rep in range(4):
+        for t in got:
+            t.fill_(-1)
+        torch.cuda.synchronize()
+        for _ in range(6):
+            many(got[0])
+            with torch.cuda.stream(side):
+                for _ in range(4):
+                    g.replay()
+        torch.cuda.synchronize()
+        for t, v in zip(got, want):
+            assert torch.equal(t, v), rep
