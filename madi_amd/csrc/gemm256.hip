@@ -335,17 +335,29 @@ f16 *gemm256_weight() {
 
 // Whole 256-column groups (a weight that fits its array, byte offsets inside
 // 2 GiB) whose tiles fill their rounds of one tile per CU to at least nine
-// tenths: a tile costs 0.87 to 0.9 of the two 128 x 256 tiles of the fused kernels (at M = 24000 1280 ->
-// 5120 + bias + GELU 351-366 -> 331-345 us, 5120 -> 1280 291-315 -> 268-283;
-// at M = 6000 1280 -> 5120 + GELU 95 -> 93), and a round that is emptier than
-// that gives it back (M = 5000, 400 tiles in two rounds, 91 -> 93 us; M =
-// 4000, 320 tiles, 71 -> 82).
+// tenths, where the kernels of gemm.hip are the slower ones (us, theirs /
+// these, back to back; the pass that writes the weight counts here):
+// - In rounds, a tile stands for two of their 128 x 256 ones, which it takes
+//   0.91 to 0.98 of, so up to a fifteenth more rounds than theirs (1280 ->
+//   5120 + bias: equal rounds M = 9200 114 / 107, 15000 186 / 171, 22000 264 /
+//   248; a fifteenth more M = 23600 278 / 275, 299 / 287, + GELU 348 / 343,
+//   319 / 324; a thirteenth more M = 21000 243 / 246, + GELU 277 / 288; a
+//   ninth more M = 14600 169 / 173, + GELU 194 / 205).
+// - At two rounds or more the weight's pass needs 5120 rows to be worth it
+//   (n x k = 8192 x 768, M = 3840 53.8 / 58.1, 6400 x 1280, M = 5120 81.1 /
+//   81.1, 5120 x 1280, M = 6000 80.9 / 77.4).
+// - One round is short: M = 3072 of 5120 x 1280 37.9 / 44.1, 12288 of 1280 x
+//   1280 38.7 / 40.8, 12288 of 1280 x 2048 56.8 / 57.4, 6144 of 2560 x 3072
+//   82.5 / 85.9; 12000 of 1280 x 5120 133 / 130, 10240 of 1536 x 5120 135 /
+//   130, 20480 of 768 x 3072 85.4 / 82.5.
 bool gemm256_suits(uint32_t m, uint32_t n, uint32_t k) {
   const uint64_t cus = (uint64_t)cu_count() / 8 * 8;
   if (n % kBN || cus == 0 || (uint64_t)n * k * 2 >= kWeightBytes || (uint64_t)n * 512 >= (1ull << 31))
     return false;
   const uint64_t tiles = (uint64_t)((m + kBM - 1) / kBM) * (n / kBN), rounds = (tiles + cus - 1) / cus;
-  return tiles * 10 >= rounds * cus * 9;
+  const uint64_t fused = (uint64_t)((m + 127) / 128) * (n / kBN), fused_rounds = (fused + cus - 1) / cus;
+  if (tiles * 10 < rounds * cus * 9 || rounds * 2 * 15 > fused_rounds * 16) return false;
+  return rounds >= 2 ? m >= 5120 : m >= 10240 && k >= 3072;
 }
 
 int gemm256(const void *a, const uint8_t *qs, const f16 *sc, void *c, const float *bias, uint32_t m,

@@ -9,9 +9,54 @@ from madi_amd import _lib, synth
 from test_gpu_q8 import TOL, dev, dev_f16, host_f16, normwise, say, tight_epi_ok, tight_ok
 
 torch = pytest.importorskip("torch")
-pytestmark = pytest.mark.gpu
 
-EPI = [O.EPI_NONE, O.EPI_BIAS, O.EPI_BIAS_GELU]
+
+def takes_256(m, n, k, cus=256):
+    """The dispatch of madi_q8_gemm (gemm.hip, gemm256.hip) up to the 256 x 256
+    tiles: whether an eager call over m rows takes them."""
+    def tiles(mt, pw=2):
+        return -(-m // (32 * mt)) * -(-n // (128 * pw))
+
+    chunks = k // 64
+    if m <= 64 or (tiles(4) < 160 and chunks >= 64 and 240 // tiles(4) > 1):
+        return False  # few rows; K split
+    if min(tiles(1), tiles(2), tiles(3)) <= cus:
+        return False  # lower tiles, one per CU
+    t, fused = -(-m // 256) * (n // 256), -(-m // 128) * (n // 256)
+    rounds, fused_rounds = -(-t // cus), -(-fused // cus)
+    if n % 256 or n * k * 2 >= 16 << 20 or n * 512 >= 1 << 31:
+        return False
+    if t * 10 < rounds * cus * 9 or rounds * 30 > fused_rounds * 16:
+        return False
+    return m >= 5120 if rounds >= 2 else m >= 10240 and k >= 3072
+
+
+# Streams (the chunks of a workgroup's tiles) of one and two chunks, of two and
+# four, three and six, four and eight, of two and three tiles; row tails of
+# one, 65, 76 and 112 rows; one tile a workgroup (K from 3072); a fifteenth more
+# rounds than the fused kernels.
+CASES = [
+    (5120, 6144, 64, O.EPI_NONE), (5121, 5888, 64, O.EPI_BIAS), (5185, 5888, 128, O.EPI_BIAS_GELU),
+    (7500, 4096, 192, O.EPI_NONE), (6000, 5120, 256, O.EPI_BIAS), (12700, 3840, 128, O.EPI_BIAS_GELU),
+    (10241, 1536, 3072, O.EPI_BIAS), (24000, 5120, 64, O.EPI_NONE), (6000, 5120, 1280, O.EPI_BIAS_GELU),
+]
+# Next to them, on the fused kernels: a row fewer, a K shorter, more rounds than
+# a fifteenth more, a round less than nine tenths full; few rows of wide
+# weights in one round (one of 256 tiles of 96 rows) and in two and three.
+OTHERS = [
+    (5119, 6144, 64, O.EPI_NONE), (10240, 1536, 3008, O.EPI_BIAS), (17700, 5120, 64, O.EPI_NONE),
+    (5888, 5120, 256, O.EPI_BIAS), (65, 65536, 64, O.EPI_NONE), (256, 59136, 128, O.EPI_BIAS),
+    (500, 29696, 192, O.EPI_BIAS_GELU), (600, 20480, 256, O.EPI_NONE),
+    (1900, 15872, 192, O.EPI_BIAS_GELU), (2305, 19456, 64, O.EPI_BIAS),
+]
+
+
+def test_cases_take_their_routes():
+    assert all(takes_256(*c[:3]) for c in CASES)
+    assert not any(takes_256(*c[:3]) for c in OTHERS)
+    # a 30 s window more or less of the encoder's MLP
+    assert [w for w in range(1, 17) if takes_256(1500 * w, 5120, 1280)] == [4, 6, 8, 10, 12, 15, 16]
+    assert [w for w in range(1, 17) if takes_256(1500 * w, 1280, 5120)] == [8, 16]
 
 
 @pytest.fixture(scope="module")
@@ -34,14 +79,8 @@ def check(c, a, qs, sc, bias, epi, rows):
     assert np.all(np.isfinite(c))
 
 
-# One tile per CU (streams of one, two, three and four chunks; row tails of 65
-# rows and more), two rounds with an uneven second one, three tiles per
-# workgroup with a row tail of one.
-@pytest.mark.parametrize("m,n,k,epi", [
-    (65, 65536, 64, O.EPI_NONE), (256, 59136, 128, O.EPI_BIAS), (500, 29696, 192, O.EPI_BIAS_GELU),
-    (600, 20480, 256, O.EPI_NONE), (1900, 15872, 192, O.EPI_BIAS_GELU), (2305, 19456, 64, O.EPI_BIAS),
-    (6000, 5120, 1280, O.EPI_BIAS_GELU),
-])
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,epi", CASES + OTHERS)
 def test_tiles_against_oracle(q, m, n, k, epi):
     say(f"gemm256 m={m} n={n} k={k} epi={epi}")
     a, qs, sc = synth.gemm_case(m + k, m, n, k)
@@ -58,12 +97,15 @@ def test_tiles_against_oracle(q, m, n, k, epi):
     edges = np.arange(128, m, 128)
     rows = np.unique(np.r_[0, 15, 16, 63, 64, m // 2, m - 2, m - 1, edges[:8] - 1, edges[:8]])
     check(host_f16(big)[:m], a, qs, sc, bias, epi, rows)
-    # again, and through the fixed scratch: the same bits
+    # again, and through the other entry point: the same bits
     for name in ("madi_q8_gemm", "madi_q8_gemm_noalloc"):
         big.fill_(0x7E00)
         call(name)
         q.sync()
         assert np.array_equal(big.cpu().numpy(), out), name
+    # which kernel ran: a captured call takes the fused ones, whose sums are in
+    # another order
+    assert np.array_equal(captured(q, call, big), out) != takes_256(m, n, k)
 
 
 def capture(q, call):
@@ -79,6 +121,16 @@ def capture(q, call):
     return g
 
 
+def captured(q, call, out):
+    """The result of a captured madi_q8_gemm, replayed once."""
+    g = capture(q, lambda: call("madi_q8_gemm"))
+    out.fill_(0x7E00)
+    g.replay()
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+@pytest.mark.gpu
 def test_captured_noalloc_is_the_captured_gemm(q):
     """Captured, the two entry points take the same kernels (the fused ones,
     which share no memory with other calls): the same bits, over replays with
@@ -114,6 +166,7 @@ def test_captured_noalloc_is_the_captured_gemm(q):
     check(host_f16(eager), a2, qs2, sc2, bias, O.EPI_BIAS, rows)
 
 
+@pytest.mark.gpu
 def test_captured_calls_share_no_scratch(q):
     """A captured call runs the fused kernels, before and after the first
     eager one: the graphs' replays, with eager calls of the same shape and
@@ -162,6 +215,7 @@ def test_captured_calls_share_no_scratch(q):
     check(host_f16(eager), a2, qs2, sc2, bias, O.EPI_BIAS_GELU, rows)
 
 
+@pytest.mark.gpu
 def test_weight_is_not_in_the_workspace(q):
     """An eager many-row call keeps its 13 MB weight out of the split-K
     workspace (4 MiB after madi_init), which captured calls use: it takes no
@@ -181,6 +235,7 @@ def test_weight_is_not_in_the_workspace(q):
         assert torch.cuda.mem_get_info()[0] == before
 
 
+@pytest.mark.gpu
 def test_replayed_split_k_beside_an_eager_call(q):
     """Split-K calls, captured, replay on a stream of their own while eager
     many-row calls run on the library's: each result keeps its bits."""
