@@ -6,14 +6,14 @@
 // share the arithmetic and the epilogues.
 //
 // q8_gemv_kernel, the vocab matrix and other wide ones (HBM-bound): a
-// workgroup of four waves owns one 32-row panel of the panel layout and its
-// waves split K.  Every wave64 load instruction moves one contiguous KiB (16
+// workgroup of four waves (sixteen for 128 to 255 panels of a long K) owns one
+// 32-row panel of the panel layout and its waves split K.  Every wave64 load instruction moves one contiguous KiB (16
 // bytes per lane, lane (h, r) receiving 16 weights of row r in quantisation
 // block h), issued as a buffer load with the panel/chunk offset in an SGPR.
 // Each wave streams its K range through a two-chunk window (use chunk c,
-// refill with chunk c+2).  62 - 71 VGPRs (seven waves per SIMD allow 72), so
-// every workgroup of the 51866-row vocab matrix (1621 panels, seven per CU)
-// is resident from the start.
+// refill with chunk c+2).  Four waves: 62 - 71 VGPRs (seven waves per SIMD
+// allow 72), so every workgroup of the 51866-row vocab matrix (1621 panels,
+// seven per CU) is resident from the start.
 //
 // q8_gemv_rows_kernel, the decoder's projections (latency-bound): a workgroup
 // owns 8 or 16 rows and all of K (below).
@@ -45,8 +45,9 @@ using namespace madi;
 namespace {
 
 // Waves per panel of the wide kernel (seven workgroups per CU), which takes
-// matrices of at least kWidePanels panels.
-constexpr int kWaves = 4;
+// matrices of at least kWidePanels panels; and of its form for fewer panels
+// of a long K, at most one workgroup per CU.
+constexpr int kWaves = 4, kLongWaves = 16;
 constexpr uint32_t kWidePanels = 256;
 // Chunks in flight per wave, a sliding window: two keeps ~26 MB of the vocab
 // matrix in flight across the GPU, enough to cover HBM latency, while the
@@ -76,10 +77,10 @@ typedef __attribute__((address_space(1))) float gfloat;
 typedef __attribute__((address_space(1))) uint32_t guint;
 inline uint64_t addr(const void *p) { return reinterpret_cast<uint64_t>(p); }
 
-// LDS bytes of the wide kernel: x (K elements of XT), the waves' partials
-template <typename XT>
+// LDS bytes of the wide kernel: x (K elements of XT), the KW waves' partials
+template <typename XT, int KW>
 constexpr size_t lds_bytes(uint32_t k) {
-  return (size_t)k * sizeof(XT) + kWaves * 32 * 4;
+  return (size_t)k * sizeof(XT) + KW * 32 * 4;
 }
 
 // One chunk's loads for a lane: its two 16-byte units and its block's scale.
@@ -222,12 +223,11 @@ __device__ inline void epi_store(float v, const RowEpi &e, uint32_t row, uint32_
 template <typename XT>
 constexpr bool kBlockF32 = sizeof(XT) == 4;
 
-// Grid: one workgroup per panel.  bias is q's for the QKV mode.
-template <typename XT, int MODE>
-__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(7))) void q8_gemv_kernel(
+// Grid: one workgroup of KW waves per panel.  bias is q's for the QKV mode.
+template <typename XT, int MODE, int KW>
+__global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(KW == kWaves ? 7 : 4))) void q8_gemv_kernel(
     uint64_t qs_, uint64_t sc_, uint64_t x_, uint32_t n, uint32_t K, uint64_t out_, uint64_t bias_,
     uint64_t vb_, uint64_t kc_, uint64_t vc_, uint64_t pos_) {
-  constexpr int KW = kWaves;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   XT *xs = reinterpret_cast<XT *>(smem);                        // [K]
   float *red = reinterpret_cast<float *>(smem + (size_t)K * sizeof(XT));  // [KW][32]
@@ -241,15 +241,21 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(7))
   const uint32_t chunks = K / kChunkK;
   const uint32_t c0 = (wave * chunks) / KW, c1 = ((wave + 1) * chunks) / KW;
 
-  // ---- The first weight window, then x (16 bytes per thread and piece), so
-  // the HBM requests leave before the L2-resident vector's (alternating runs
-  // in one process: 12.16 -> 11.92 us with f16 x, 12.66 -> 12.35 us with f32
-  // x).  Lanes past a partial panel's last row read row R-1 (in bounds; their
-  // sums are never stored).
+  // ---- Four waves: the first weight window, then x (16 bytes per thread and
+  // piece), so the HBM requests leave before the L2-resident vector's
+  // (alternating runs in one process: 12.16 -> 11.92 us with f16 x, 12.66 ->
+  // 12.35 us with f32 x).  Sixteen: x first, whose staging barrier is then the
+  // longer wait.  Lanes past a partial panel's last row read row R-1 (in
+  // bounds; their sums are never stored).
+  constexpr bool kWeightsFirst = KW == kWaves;
   const uint32_t pieces = K * sizeof(XT) / 16;
   const rsrc_t xr = make_rsrc((const void *)x_, K * sizeof(XT));
   u32x4 xv0 = {}, xv1 = {};
   const uint32_t i0 = threadIdx.x, i1 = threadIdx.x + KW * 64;
+  if constexpr (!kWeightsFirst) {
+    if (i0 < pieces) xv0 = __builtin_amdgcn_raw_buffer_load_b128(xr, i0 * 16, 0, 0);
+    if (i1 < pieces) xv1 = __builtin_amdgcn_raw_buffer_load_b128(xr, i1 * 16, 0, 0);
+  }
   const rsrc_t wq = make_rsrc((const void *)qs_, n * K), ws = make_rsrc((const void *)sc_, n * (K / 32) * 2);
   // chunks past the wave's range load through an empty resource: no memory
   // access, zeros returned, so their scale is 0 and they add exactly nothing.
@@ -267,8 +273,10 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(7))
     const bool in = c0 + k < c1;
     load_chunk(win[k], in ? wq : wz, in ? ws : wz, K, c0 + k, p, R, w_voff, s_voff);
   }
-  if (i0 < pieces) xv0 = __builtin_amdgcn_raw_buffer_load_b128(xr, i0 * 16, 0, 0);
-  if (i1 < pieces) xv1 = __builtin_amdgcn_raw_buffer_load_b128(xr, i1 * 16, 0, 0);
+  if constexpr (kWeightsFirst) {
+    if (i0 < pieces) xv0 = __builtin_amdgcn_raw_buffer_load_b128(xr, i0 * 16, 0, 0);
+    if (i1 < pieces) xv1 = __builtin_amdgcn_raw_buffer_load_b128(xr, i1 * 16, 0, 0);
+  }
 
   // lanes 0..R-1 of wave 0 own the panel's rows
   const uint32_t erow = p * kPanelRows + threadIdx.x;
@@ -287,7 +295,35 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(7))
   // registers with chunk c + kWin
   float acc = 0.0f;
   uint32_t cfirst = c0;
-  if constexpr (kBlockF32<XT>) {
+  if constexpr (KW == kLongWaves) {
+    // Sixteen waves: the first window's activations are read from LDS now,
+    // while its weights are still in flight, instead of after they land, when
+    // all the waves would queue at the LDS at once.
+    if (c0 < c1) {
+      XT xf[kWin][32];
+#pragma unroll
+      for (int k = 0; k < kWin; ++k) {
+        const uint32_t cc = c0 + k < c1 ? c0 + k : c1 - 1;
+#pragma unroll
+        for (int i = 0; i < 32; ++i) xf[k][i] = xs[cc * kChunkK + h * 32 + i];
+      }
+      // the reads stay ahead of the first wait for the weights
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < kWin; ++k) {
+        // (a chunk past the range adds nothing where x is infinite either)
+        const float before = acc;
+        accumulate_x<XT>(win[k], xf[k], acc);
+        acc = c0 + k < c1 ? acc : before;
+        const uint32_t cn = c0 + k + kWin;
+        const bool in = cn < c1;
+        load_chunk(win[k], in ? wq : wz, in ? ws : wz, K, cn, p, R, w_voff, s_voff);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      cfirst = c0 + kWin < c1 ? c0 + kWin : c1;
+    }
+  }
+  if constexpr (KW == kWaves && kBlockF32<XT>) {
     // The vocab matrix with fp32 activations: each unit's activations are
     // read from LDS one unit ahead of their use (the next chunk's first unit
     // during this chunk's second), so the LDS latency passes under the
@@ -318,8 +354,11 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(7))
     }
     cfirst = c1;
   }
+  // whole windows, then (sixteen waves) the last one's chunks by themselves:
+  // a slot past the range adds nothing there even where x is infinite
+  const uint32_t cend = KW == kLongWaves ? c1 - (c1 - cfirst) % kWin : c1;
 #pragma unroll 1
-  for (uint32_t c = cfirst; c < c1; c += kWin) {
+  for (uint32_t c = cfirst; c < cend; c += kWin) {
 #pragma unroll
     for (int k = 0; k < kWin; ++k) {
       // a chunk past the range (zeros, scale 0) reads the x of the range's
@@ -333,6 +372,11 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(7))
       // slots would have to land before either is reissued
       __builtin_amdgcn_sched_barrier(0);
     }
+  }
+  if constexpr (KW == kLongWaves) {
+#pragma unroll
+    for (int k = 0; k < kWin - 1; ++k)
+      if (cend + k < c1) accumulate<XT>(win[k], cend + k, xs, h, acc);
   }
 
   acc += __shfl_xor(acc, 32);
@@ -574,6 +618,22 @@ void pick_rows(const GemvArgs &a) {
   else launch_rows<XT, MODE, NR, 3, false>(a);
 }
 
+template <typename XT, int MODE, int KW>
+void launch_panels(const GemvArgs &a, uint32_t np) {
+  hipLaunchKernelGGL((q8_gemv_kernel<XT, MODE, KW>), dim3(np), dim3(KW * 64), (lds_bytes<XT, KW>(a.k)),
+                     stream(), addr(a.qs), addr(a.sc), addr(a.x), a.n, a.k, addr(a.out),
+                     addr(MODE == kQkv ? a.qb : a.bias), addr(a.vb), addr(a.kc), addr(a.vc), addr(a.pos));
+}
+
+// From 128 panels of a K past 1536 sixteen waves per panel are the faster
+// form: 16 rows per workgroup would be 256 workgroups and more, which hold a
+// CU each at the registers and waves of a long K, in two rounds, each staging
+// all of x.  (Issued from C, us, 16 waves per panel / 16 rows: 4608 x 1536
+// 3.6 / 3.5, x 1920 3.8 / 4.0, x 3072 5.4 / 6.1, x 4096 5.8 / 9.4, 5120 x 5120
+// 7.3 / 11.1, 8160 x 1280 4.0 / 3.9, x 2048 5.2 / 5.5, x 6144 10.9 / 14.6;
+// 4064 x 4096, in four splits then, 10.3 / 6.3.)
+constexpr uint32_t kLongPanels = 128, kLongK = 1536;
+
 template <typename XT, int MODE>
 int launch(const char *what, const GemvArgs &a) {
   if (!a.out || !a.x || !a.qs || !a.sc) return fail(MADI_ERR_NULL, "%s: null pointer", what);
@@ -604,9 +664,9 @@ int launch(const char *what, const GemvArgs &a) {
   }
   const uint32_t np = (a.n + kPanelRows - 1) / kPanelRows;
   if (np >= kWidePanels)
-    hipLaunchKernelGGL((q8_gemv_kernel<XT, MODE>), dim3(np), dim3(kWaves * 64), lds_bytes<XT>(a.k), stream(),
-                       addr(a.qs), addr(a.sc), addr(a.x), a.n, a.k, addr(a.out),
-                       addr(MODE == kQkv ? a.qb : a.bias), addr(a.vb), addr(a.kc), addr(a.vc), addr(a.pos));
+    launch_panels<XT, MODE, kWaves>(a, np);
+  else if (np >= kLongPanels && a.k > kLongK)
+    launch_panels<XT, MODE, kLongWaves>(a, np);
   else if (a.n > kRows8)
     pick_rows<XT, MODE, 2>(a);
   else

@@ -1,6 +1,7 @@
 """The decoder GEMV's row-group kernel (madi_amd/csrc/gemv.hip: 8 or 16 rows
-of all of K per workgroup) at the edges of its ranges, against the exact
-product within fp32 accumulation."""
+of all of K per workgroup) at the edges of its ranges, and the sixteen waves
+per panel that take 128 to 255 panels of a longer K, against the exact product
+within fp32 accumulation."""
 import numpy as np
 import pytest
 
@@ -23,10 +24,14 @@ def q():
 # rows: one, a partial and a whole group, a last panel of one and of nine rows,
 # the largest of 8 rows a workgroup and the next, the last narrow width and
 # the first wide one; K: one chunk, odd counts, the most of one pair a wave
-# (32 chunks) and the next, the most in flight at once (96) and beyond
+# (32 chunks) and the next, the most in flight at once (96) and beyond.
+# Sixteen waves per panel: the first and last panel count, both sides of K =
+# 1536, odd chunk counts, one window per wave (32 chunks) and more.
 @pytest.mark.parametrize("n,k", [
     (1, 64), (7, 64), (8, 128), (9, 192), (33, 320), (41, 2048), (26, 2112), (2304, 192), (2305, 192),
     (2311, 2112), (8160, 128), (8161, 128), (40, 6144), (40, 6208), (2344, 6272), (17, 12288),
+    (4064, 1600), (4065, 1600), (4065, 1536), (4100, 2048), (5120, 2112), (8160, 3136), (8161, 1600),
+    (4096, 12288),
 ])
 def test_rows_against_exact(q, n, k):
     say(f"gemv rows n={n} k={k}")
@@ -86,11 +91,11 @@ def test_rows_qkv(q, d):
 def test_rows_infinite_x(q):
     """A missing chunk (an odd count, a window's pairs past the range) adds
     nothing even where the activations it stands in for are infinite."""
-    for n, k in ((16, 192), (16, 5120)):
+    for n, k in ((16, 192), (16, 5120), (4096, 1600), (4096, 3136)):
         x16, qs, sc = synth.gemv_case(3, n, k)
         x = x16.astype(np.float32)
         x[-3] = np.inf
-        qs[:, -3] = 1 + np.arange(n)
+        qs[:, -3] = 1 + np.arange(n) % 100
         w = q.upload_q8(qs, sc)
         out = torch.empty(n, dtype=torch.float32, device="cuda")
         q.kGemvQ8(out, dev(x), w, n, k)
