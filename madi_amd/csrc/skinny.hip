@@ -584,12 +584,20 @@ int launch_skinny16(const Proj &a) {
 // / 64 rows 3.35 / 2.64, 3.75 / 2.88, 4.42 / 3.72, 4.48 / 3.88, 3840 x 1280 at
 // 8 / 16 / 32 rows 3.43 / 2.92, 3.87 / 3.19, 4.51 / 4.17; past that the
 // activations, which every workgroup loads, cost more (5120 x 1280 at 8 / 32
-// rows 3.47 / 3.53, 4.6 / 5.7, 2560 x 1280 at 64 4.5 / 5.4).  A long K on few
-// panels, which the panel kernel splits over workgroups that meet through
-// memory, only up to 8 rows (1280 x 5120 at 8 / 16 rows 6.11 / 4.83, 6.5 / 6.9).
+// rows 3.47 / 3.53, 4.6 / 5.7, 2560 x 1280 at 64 4.5 / 5.4).
+// In K: more than 16 rows, while one round of loads holds it (24 chunks: 2048
+// x 1536 at 32 rows 4.5 / 4.4, x 1600 5.2 / 5.9, x 2048 6.5 / 6.6, 4096 x 2048
+// 6.4 / 7.2); up to 16 rows, to 2048 (1280 x 2048 at 16 rows 5.5 / 4.5).  A
+// longer K on fewer than 128 panels, which the panel kernel splits over
+// workgroups that meet through memory, only up to 8 rows (1280 x 5120 at 8 /
+// 16 rows 6.11 / 4.83, 6.5 / 6.9) and, where its four splits are one round of
+// workgroups (2048 rows of weight), up to 5120 (2048 x 5120 at 8 rows 6.7 /
+// 5.4, x 6144 7.1 / 7.5, 1280 x 12288 9.4 / 12.7, 2176 x 12288 15.8 / 13.4).
 bool skinny16_suits(uint32_t m, uint32_t n, uint32_t k) {
   const uint64_t wgs = (uint64_t)((n + 15) / 16) * ((m + kSlice - 1) / kSlice);
-  return wgs <= (uint64_t)cu_count() && (k <= 2048 || (m <= 8 && n < 128 * kPanelRows));
+  if (wgs > (uint64_t)cu_count()) return false;
+  if (m > 16) return k <= kRowsWaves * kRowsWin * kChunkK;
+  return k <= 2048 || (m <= 8 && n < 128 * kPanelRows && (n > 2048 || k <= 5120));
 }
 
 // Launch shapes.  Single panels (decoder projections, 40 - 160 panels): eight

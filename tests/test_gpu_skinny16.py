@@ -25,12 +25,15 @@ def q():
 # activation rows: one, the edges of the 8-, 16- and 32-row forms, a second
 # slice of one row and several; weight rows: less than a group, a last panel
 # of 1, 9, 17 and 26 rows, one workgroup per CU and one more, wider; K: one chunk, odd
-# counts, one window per wave (24 chunks) and the next, the routes' line at
-# 2048, long ones (80 and 81 chunks)
+# counts, one window per wave (24 chunks) and the next, the routes' lines at
+# 1536 (more than 16 rows), 2048 and 5120 (up to 2048 weight rows), long ones
+# (80 and 81 chunks)
 @pytest.mark.parametrize("m,n,k", [
     (1, 7, 64), (8, 16, 128), (9, 33, 192), (16, 41, 1536), (17, 49, 1600), (32, 90, 1280), (33, 40, 320),
     (100, 26, 704), (16, 4096, 64), (16, 4097, 64), (9, 3840, 1280), (8, 8192, 128), (8, 1280, 2048),
     (8, 1280, 2112), (5, 1281, 5120), (8, 300, 5184), (9, 300, 5184), (320, 384, 384),
+    (17, 49, 1536), (33, 200, 1536), (16, 49, 1600), (16, 49, 2048), (17, 49, 2048), (8, 2048, 5120),
+    (8, 2048, 5184), (8, 2049, 5184), (3, 640, 12288),
 ])
 def test_rows_against_exact(q, m, n, k):
     say(f"skinny16 m={m} n={n} k={k}")
