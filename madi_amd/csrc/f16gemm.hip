@@ -78,17 +78,17 @@ __device__ inline f16x4 lds_read_tr(uint32_t addr) {
 __device__ inline uint32_t swz_a(uint32_t row) { return (row >> 1) & 7; }
 // buffer cache policy sc1: a store writes through the XCD's L2
 constexpr int kSc1 = 16;
+constexpr uint32_t kGroupM = 6;  // row tiles per group (below)
 __device__ inline uint32_t swz_b(uint32_t row) { return (row & 3) << 2; }
 
 // Grid: one workgroup per tile, the grid rounded up to a multiple of 8.
 // Workgroups x and x + 8 run on the same XCD (round-robin dispatch), so each
-// XCD takes a contiguous run of tiles, walked in groups of group_m row tiles
-// with column tiles outermost, and the operands of a run are fetched into one
-// L2.  Up to 12 row tiles are one group; more go in sixes, so that a run is
-// nearly square: 30 tiles of 64 x 128 over all 24 row tiles of 1500 rows read
-// the whole of A into every L2 (5120 -> 1280 30.8 -> 27.9 us, 1280 -> 1280 + bias
-// 9.8 -> 9.2, 1000 rows of 5120 -> 1280 27.3 -> 24.4; groups of 3, 4, 8 28.6,
-// 29.2, 28.8).  M rows past the last are read
+// XCD takes a contiguous run of tiles, column tiles outermost, and the B
+// columns of a run are fetched into one L2.  GROUPS: the run is walked in
+// groups of six row tiles, so that it is nearly square: 30 tiles of 64 x 128
+// over all 24 row tiles of 1500 rows read the whole of A into every L2 (groups
+// of 3, 4, 6, 8 of 1500 x 5120 -> 1280 28.6, 29.2, 27.9, 28.8 us, none 30.8;
+// where: grouped below).  M rows past the last are read
 // as the last row (in bounds) and never stored.  Requires K % 64 == 0,
 // N % BN == 0, A, B, C and bias 16-byte aligned.  F32O: C is f32 (the
 // unrounded sums, no epilogue) instead of f16.
@@ -101,11 +101,10 @@ __device__ inline uint32_t swz_b(uint32_t row) { return (row & 3) << 2; }
 // per chunk: the producers arrive once their DMAs of the chunk about to be
 // computed have landed (vmcnt), the computing waves once they are done
 // reading the chunk before, whose stage the producers refill right after.
-template <class G, int EPI, bool F32O>
+template <class G, int EPI, bool F32O, bool GROUPS>
 __global__ __launch_bounds__(512) void f16_nn_gemm_kernel(
     const f16 *__restrict__ A, const f16 *__restrict__ B, uint32_t M, uint32_t N, uint32_t K,
-    uint32_t tiles_m, uint32_t tiles_n, uint32_t tiles, uint32_t group_m, void *__restrict__ C,
-    const float *__restrict__ bias) {
+    uint32_t tiles_m, uint32_t tiles, void *__restrict__ C, const float *__restrict__ bias) {
   constexpr int S = G::kStages, BN = G::BN, TMw = G::kTM, TNw = G::kTN, WNw = G::kWN;
   static_assert(!F32O || EPI == MADI_EPI_NONE, "the f32 result takes no epilogue");
   constexpr uint32_t kOut = F32O ? 4 : 2;  // bytes per C element
@@ -120,11 +119,11 @@ __global__ __launch_bounds__(512) void f16_nn_gemm_kernel(
   if (slot >= per + (x < extra ? 1u : 0u)) return;
   const uint32_t item = x * per + (x < extra ? x : extra) + slot;
   uint32_t first_m = 0, in = item, gm = tiles_m;
-  if (group_m < tiles_m) {
-    const uint32_t per_group = group_m * tiles_n, gi = item / per_group;
-    first_m = gi * group_m;
+  if constexpr (GROUPS) {
+    const uint32_t per_group = kGroupM * (N / BN), gi = item / per_group;
+    first_m = gi * kGroupM;
     in = item - gi * per_group;
-    gm = tiles_m - first_m < group_m ? tiles_m - first_m : group_m;
+    gm = tiles_m - first_m < kGroupM ? tiles_m - first_m : kGroupM;
   }
   const uint32_t tn = in / gm, tm = first_m + (in - tn * gm);
   const uint32_t m0 = tm * G::BM, n0 = tn * BN, nk = K / 64;
@@ -373,14 +372,39 @@ bool nn_ok(const void *a, const void *b, const void *c, const float *bias, uint3
          (uint64_t)k * n * 2 < (1ull << 31) && (uint64_t)n * 128 * 4 < (1ull << 31);
 }
 
+// Whether tiles of bm rows are walked in groups: where the A rows that the
+// ungrouped run of an XCD covers do not fit its 4 MiB L2, and there are enough
+// row tiles.  Ungrouped / grouped, us:
+// - 64-row tiles, more than 768 rows: 1500 x 1280 -> 1280 (3.8 MB) 9.3 / 8.9,
+//   1500 x 5120 -> 1280 30.6 / 27.5, 1000 x 5120 -> 1280 27.5 / 24.7, 4500 x
+//   2048 -> 512 28.3 / 22.4; 1408 x 1280 -> 1280 (3.6 MB) 8.8 / 8.8, 1024 x
+//   1280 -> 1280 7.9 / 8.3, 1537 x 1536 -> 384 (3 column tiles, so a run is a
+//   third of the rows) 8.0 / 8.6.
+// - 128 x 128 tiles, more than 1920 rows: 2305 x 1280 -> 1280 12.6 / 11.5, 3000
+//   14.5 / 13.1; 1700 x 1280 -> 2560 24.2 / 24.7.
+// - 128 x 256 tiles, more than 3584 rows: 4500 x 1280 -> 5120 72.5 / 69.0, 6000
+//   x 1280 -> 3840 73.1 / 69.5; 2305 x 1280 -> 3840 40.1 / 41.5, 3073 x 1280 ->
+//   5120 46.3 / 47.6.
+// The group arithmetic is an instance of its own: in the ungrouped kernel it
+// cost 2 to 10 % (1 x 5120 -> 1280 18.9 / 20.7).
+template <class G>
+bool grouped(uint32_t m, uint32_t n, uint32_t k, uint32_t tiles) {
+  const uint32_t least = G::BM == 64 ? 768 : G::BN == 128 ? 1920 : 3584;
+  const uint64_t rows = (uint64_t)tiles * G::BM / 8 < m ? (uint64_t)tiles * G::BM / 8 : m;
+  return m > least && n > (uint32_t)G::BN && rows * k * 2 > 3700000;
+}
+
 template <class G, int EPI, bool F32O = false>
 int launch_nn(const void *a, const void *b, void *c, const float *bias, uint32_t m, uint32_t n,
               uint32_t k, const char *what) {
   const uint32_t tiles_m = (m + G::BM - 1) / G::BM, tiles = tiles_m * (n / G::BN);
-  const uint32_t group_m = tiles_m > 12 ? 6 : tiles_m;
-  hipLaunchKernelGGL((f16_nn_gemm_kernel<G, EPI, F32O>), dim3((tiles + 7) & ~7u), dim3(512), 0,
-                     stream(), static_cast<const f16 *>(a), static_cast<const f16 *>(b), m, n, k,
-                     tiles_m, n / G::BN, tiles, group_m, c, bias);
+  const auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((tiles + 7) & ~7u), dim3(512), 0, stream(),
+                       static_cast<const f16 *>(a), static_cast<const f16 *>(b), m, n, k, tiles_m, tiles,
+                       c, bias);
+  };
+  if (grouped<G>(m, n, k, tiles)) go(f16_nn_gemm_kernel<G, EPI, F32O, true>);
+  else go(f16_nn_gemm_kernel<G, EPI, F32O, false>);
   return check_launch(what);
 }
 

@@ -1,6 +1,7 @@
-"""The F16-weight GEMM's tile order (madi_amd/csrc/f16gemm.hip): more than 12
-row tiles are walked in groups of six, a last group that is not whole among
-them; every tile is computed once."""
+"""The F16-weight GEMM's tile order (madi_amd/csrc/f16gemm.hip): row tiles are
+walked in groups of six, a last group that is not whole among them, where
+their A rows do not fit an L2, and column by column elsewhere; every tile is
+computed once."""
 import numpy as np
 import pytest
 
@@ -11,7 +12,14 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("m,n,k", [(768, 128, 64), (769, 256, 128), (1153, 384, 64), (1500, 1280, 128)])
+# ungrouped; then in groups: 64 x 128 tiles (13 row tiles, 24, 25), 128 x 128
+# (16, 19), 128 x 256 (29, 33); and the last shape of each before its line
+@pytest.mark.parametrize("m,n,k", [
+    (768, 128, 64), (769, 256, 128), (1153, 384, 64), (1500, 1280, 128),
+    (769, 1280, 5120), (1500, 1280, 1280), (1537, 1280, 1280), (1921, 1280, 1280), (2305, 1280, 1280),
+    (3585, 2048, 640), (4100, 1536, 1024), (768, 1280, 5120), (1408, 1280, 1280), (1920, 1408, 1280),
+    (3584, 2048, 640),
+])
 def test_groups_of_row_tiles(m, n, k):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
