@@ -54,7 +54,10 @@ OTHERS = [
 def test_cases_take_their_routes():
     assert all(takes_256(*c[:3]) for c in CASES)
     assert not any(takes_256(*c[:3]) for c in OTHERS)
-    # a 30 s window more or less of the encoder's MLP
+    # the persistent tile loop's own shapes (test_gpu_q8.py)
+    assert not any(takes_256(*c) for c in ((21000, 5120, 768), (21000, 5120, 1280), (14600, 5120, 1280),
+                                           (5500, 5120, 1280), (7001, 4096, 768), (13300, 1280, 2048)))
+    # windows of 1500 rows, the encoder's MLP
     assert [w for w in range(1, 17) if takes_256(1500 * w, 5120, 1280)] == [4, 6, 8, 10, 12, 15, 16]
     assert [w for w in range(1, 17) if takes_256(1500 * w, 1280, 5120)] == [8, 16]
 

@@ -200,7 +200,7 @@ def test_gemm_k_loop_shapes(q, m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k", [
-    (257, 1280, 5120),  # 64-row tiles: 25 tiles x 4 K splits of 20 chunks, M tail
+    (257, 1280, 5120),  # 64 x 128 tiles: 50 tiles x 4 K splits of 20 chunks, M tail
     (20, 512, 4096),    # 32-row tiles, 2 tiles x 4 splits of 16 chunks
     (64, 768, 6144),    # 64-row tiles, 3 tiles x 4 splits of 24 chunks
     (130, 512, 4288),   # 67 chunks: 4 splits of 16-17 chunks (padded loop)
@@ -422,9 +422,9 @@ def test_gemm_narrow_tiles_match_wide(q, m, n, k, epi):
 
 @pytest.mark.parametrize("name,n,k", [("fc1", 5120, 1280), ("fc2", 1280, 5120)])
 def test_gemm_long_audio_full_m(q, name, n, k):
-    """16 stacked windows, M = 24000: 128-row tiles, 188 x 20 (fc1) and 188 x 5
-    (fc2) of them, several per CU; fc2's 80-chunk K runs unsplit and
-    unpadded.  Row sample over tile boundaries, the tail and random rows."""
+    """16 stacked windows, M = 24000: 256-row tiles, 94 x 20 (fc1) and 94 x 5
+    (fc2) of them, several per CU.  Row sample over tile boundaries, the tail
+    and random rows."""
     say(f"gemm long audio {name} m=24000 n={n} k={k}")
     m = 24000
     rng = np.random.default_rng(24000 + n)
@@ -440,16 +440,21 @@ def test_gemm_long_audio_full_m(q, name, n, k):
 
 
 @pytest.mark.parametrize("m,n,k,epi", [
-    (24000, 5120, 1280, O.EPI_NONE),       # long-audio fc1: 3760 tiles, 14.7 per workgroup
+    (24000, 5120, 1280, O.EPI_NONE),       # long-audio fc1: 94 x 20 tiles of 256 x 256, 7.3 per workgroup
     (24000, 5120, 1280, O.EPI_BIAS_GELU),  # ... with bias + GELU
+    (21000, 5120, 768, O.EPI_NONE),        # 128 x 256 tiles from here on: 3300, 12.9 per workgroup
+    (21000, 5120, 1280, O.EPI_BIAS),
+    (14600, 5120, 1280, O.EPI_BIAS_GELU),  # 2300: 8.98 per workgroup, 4 short of whole rounds
+    (5500, 5120, 1280, O.EPI_NONE),        # 860: three rounds and a third of one, M tail of 124 rows
     (7001, 4096, 768, O.EPI_BIAS_GELU),    # 12-chunk K (first trip, one middle, last), M tail of 89 rows
     (13300, 1280, 2048, O.EPI_BIAS),       # 520 tiles: two rounds and 8 tiles, 32-chunk K, M tail of 116
 ])
 def test_gemm_persistent(q, m, n, k, epi):
     """At least two rounds of 128 x 256 tiles: the persistent tile loop
-    (q8_gemm_persist_kernel) issues each next tile's loads before the
-    finished tile's epilogue.  Row sample over tile boundaries and the tail;
-    a second run gives the same bits."""
+    (q8_gemm_persist_kernel), or the 256 x 256 tiles where those fill their
+    rounds, issues each next tile's loads before the finished tile's epilogue.
+    Row sample over tile boundaries and the tail; a second run gives the same
+    bits."""
     say(f"gemm persistent m={m} n={n} k={k} epi={epi}")
     rng = np.random.default_rng(m + n)
     a = synth.activations(rng, m, k)
@@ -487,15 +492,12 @@ def test_gemm_large_m(q):
 
 
 # ------------------------------------------------------------------ GEMV
-# (51866, 1280): four waves per panel; the others sixteen: (3840, 1280),
-# (5120, 1280), (40, 64) one or two chunks per wave, (1280, 5120) four K
-# splits, (5120, 4096) four chunks per wave through the two-chunk window,
-# (40, 12288) the largest K in four splits of 48 chunks
-# Shapes: the vocab and the decoder projections; 40 panels at K = 64 (one
-# chunk: fifteen of the sixteen waves own none); 5120 x 4096 (four chunks per
-# wave, past the first window); 40 x 12288 (K split over workgroups); and
-# wide matrices (256 or more panels, four waves, the fp32 vector read one
-# unit ahead) at K = 64 and 192, where some waves own no chunk and others one.
+# Shapes: the vocab (four waves per panel) and the decoder projections (8 or 16
+# rows per workgroup, a long K in one workgroup); 40 rows at K = 64 (one chunk,
+# half a pair) and at K = 12288, the largest (two rounds of the waves); 5120 x
+# 4096 (sixteen waves per panel, four chunks each, past the first window); and
+# wide matrices (256 or more panels, four waves, the fp32 vector read one unit
+# ahead) at K = 64 and 192, where some waves own no chunk and others one.
 @pytest.mark.parametrize("n,k", [(51866, 1280), (3840, 1280), (1280, 5120), (5120, 1280), (40, 64),
                                  (5120, 4096), (40, 12288), (8200, 64), (8192, 192)])
 def test_gemv_parity(q, n, k):
@@ -593,7 +595,7 @@ def test_logit_gemv_vocab(q):
     assert int(np.argmax(got)) == int(np.argmax(ref))
 
 
-@pytest.mark.parametrize("n,k", [(5120, 1280), (1280, 5120)])  # the second splits K over workgroups
+@pytest.mark.parametrize("n,k", [(5120, 1280), (1280, 5120)])  # 16 and 8 rows per workgroup
 @pytest.mark.parametrize("epi", ["bias", "gemv_q8_bias_gelu", "gemv_q8_bias_res"])
 def test_gemv_epilogues(q, epi, n, k):
     x16, qs, sc = synth.gemv_case(7, n, k)
@@ -926,17 +928,17 @@ def test_graph_replay_after_workspace_growth(q):
     rng = np.random.default_rng(37)
     qs1, sc1 = synth.q8_weight(rng, 1280, 5120)     # FFN down: four K splits
     w1 = q.upload_q8(qs1, sc1)
-    x = dev(rng.standard_normal((8, 5120)).astype(np.float32))
+    x = dev(rng.standard_normal((16, 5120)).astype(np.float32))
     xv = dev(rng.standard_normal(5120).astype(np.float32))
     a = dev_f16(synth.activations(rng, 20, 4096))
     qs2, sc2 = synth.q8_weight(rng, 512, 4096)      # 2 tiles x 4 K splits
     w2 = q.upload_q8(qs2, sc2)
-    o1 = torch.empty((8, 1280), dtype=torch.float32, device="cuda")
+    o1 = torch.empty((16, 1280), dtype=torch.float32, device="cuda")
     o2 = torch.empty(1280, dtype=torch.float32, device="cuda")
     c = torch.empty((20, 512), dtype=torch.int16, device="cuda")
 
     def seq():
-        q.pproj(x, w1, o1, 8, 1280, 5120)
+        q.pproj(x, w1, o1, 16, 1280, 5120)  # (up to 8 rows would not split)
         q.kGemvQ8(o2, xv, w1, 1280, 5120)
         q.kGemmQ8(a, w2, c, 20, 512, 4096)
 
@@ -1214,8 +1216,8 @@ def test_f16_nn_gemm_leaves_other_rows(q):
 
 def test_stream_switch_orders_split_k(q):
     """madi_set_stream makes the new stream wait for the work already issued
-    on the old one.  Split-K launches (the FFN-down GEMV 5120 -> 1280, four K
-    splits, and the GEMM 1000 x 5120 -> 1280, three K splits through the
+    on the old one.  Split-K launches (the FFN-down projection 5120 -> 1280 of
+    16 rows, four K splits, and the GEMM 1000 x 5120 -> 1280, three K splits through the
     workspace) go to two streams in turn while the first is still busy with
     twenty such GEMMs.  They share the workspace's partials and arrival
     counters one after the other, so every output equals its single-stream
@@ -1225,13 +1227,13 @@ def test_stream_switch_orders_split_k(q):
     rng = np.random.default_rng(41)
     qs1, sc1 = synth.q8_weight(rng, 1280, 5120)
     w1 = q.upload_q8(qs1, sc1)
-    xs = [dev(rng.standard_normal(5120).astype(np.float32)) for _ in range(4)]
+    xs = [dev(rng.standard_normal((16, 5120)).astype(np.float32)) for _ in range(4)]
     a = dev_f16(synth.activations(rng, 1000, 5120))
     c = torch.empty((1000, 1280), dtype=torch.int16, device="cuda")
-    outs = [torch.empty(1280, dtype=torch.float32, device="cuda") for _ in range(4)]
+    outs = [torch.empty((16, 1280), dtype=torch.float32, device="cuda") for _ in range(4)]
     q.init()
     for x, o in zip(xs, outs):
-        q.kGemvQ8(o, x, w1, 1280, 5120)
+        q.pproj(x, w1, o, 16, 1280, 5120)
     q.kGemmQ8(a, w1, c, 1000, 1280, 5120)
     q.sync()
     want, want_c = [o.clone() for o in outs], c.clone()
@@ -1244,13 +1246,13 @@ def test_stream_switch_orders_split_k(q):
         q.init(s1)
         for _ in range(20):
             q.kGemmQ8(a, w1, c, 1000, 1280, 5120)
-        q.kGemvQ8(outs[0], xs[0], w1, 1280, 5120)
-        q.kGemvQ8(outs[1], xs[1], w1, 1280, 5120)
+        q.pproj(xs[0], w1, outs[0], 16, 1280, 5120)
+        q.pproj(xs[1], w1, outs[1], 16, 1280, 5120)
         q.init(s2)
-        q.kGemvQ8(outs[2], xs[2], w1, 1280, 5120)
+        q.pproj(xs[2], w1, outs[2], 16, 1280, 5120)
         q.kGemmQ8(a, w1, c, 1000, 1280, 5120)
         q.init(s1)
-        q.kGemvQ8(outs[3], xs[3], w1, 1280, 5120)
+        q.pproj(xs[3], w1, outs[3], 16, 1280, 5120)
         torch.cuda.synchronize()
         for i, (o, w) in enumerate(zip(outs, want)):
             assert torch.equal(o, w), (rep, i)

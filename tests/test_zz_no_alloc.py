@@ -44,7 +44,7 @@ def run(q, name, a_d, w, bias_d, m, n, k, epi):
 
 # (m, n, k, epilogue): 1000 x 5120 -> 1280 + bias (80 tiles of 64 x 256,
 # three K splits: 15.7 MB of partials), then smaller split shapes (four
-# splits over 25 and 2 tiles), then a shape that does not split at all, and
+# splits over 50 and 2 tiles), then a shape that does not split at all, and
 # fc2 + bias at M = 1500, whose K split stays inside the workgroup (no scratch)
 CASES = [(1000, 1280, 5120, _lib.EPI_BIAS), (257, 1280, 5120, _lib.EPI_NONE),
          (20, 512, 4096, _lib.EPI_BIAS_GELU), (96, 512, 1280, _lib.EPI_BIAS_GELU),
@@ -119,7 +119,7 @@ def test_noalloc_under_graph_capture(q):
         torch.cuda.synchronize()
         assert np.array_equal(c.cpu().numpy(), want), rep
         # eager work between replays: smaller split shapes through the same
-        # scratch (257 rows: four splits over 25 tiles) and the workspace
+        # scratch (257 rows: four splits over 50 tiles) and the workspace
         a2, qs2, sc2 = synth.gemm_case(57 + rep, 257, 1280, 5120)
         w2 = q.upload_q8(qs2, sc2)
         a2_d = dev_f16(a2)
