@@ -2,18 +2,21 @@
 // 256 x 256 tiles on a weight dequantised once per call.
 //
 // Under a sustained MFMA load the card holds its power, not its clock: over a
-// long recording the fused kernels of gemm.hip run at 1.5 GHz with the matrix
-// pipes 66 % busy, so what pays is less energy per product.  Three things do
-// that here.  The panel-layout weight is written once per call as F16 [N][K]
+// long recording the fused kernels of gemm.hip run at 1.5 - 1.7 GHz with the
+// matrix pipes 61 - 66 % busy (5120 -> 1280), so what pays is less energy per
+// product.  Three things do that here.  The panel-layout weight is written once per call as F16 [N][K]
 // rows into an array of the library (the exact fp16_rne(q * s) of every other
 // kernel, 6.4 us for 5120 x 1280) instead of being dequantised once per 128-row
 // tile beside the MFMAs.  The MFMA is 16x16x32: a register-only loop on random
 // operands sustains 1.91 PFLOP/s with it and 1.58-1.68 with 32x32x16 (both
 // 2.4 on zeros), because each product updates half as many accumulators.  And
 // a 256 x 256 tile brings a third less through L2 and LDS per product than a
-// 128 x 256 one.  At M = 24000, 5120 -> 1280 the clock is 1.90 GHz, the matrix
-// pipes 62 % busy, 268-283 us against 291-315; without any operand loads
-// (results discarded) the same loop takes 239.
+// 128 x 256 one.  At M = 24000, 5120 -> 1280 the clock is 1.90 - 1.94 GHz, the
+// matrix pipes 62 % busy, 251-283 us against 265-315 over boxes (alternating
+// on one, 257 / 268); without any operand loads (results discarded) the same
+// loop took 239 where it took 268.  1280 -> 5120 + bias + GELU: 336 / 343 on
+// one box, 336 / 321 on another, 331-377 in all: GELU runs with nothing under
+// it (pipes 44 % busy).
 //
 // Rows past M load as zeros; results differ from the fused kernels' only by
 // the order of the fp32 sums.

@@ -590,7 +590,8 @@ int launch_skinny16(const Proj &a) {
 // 6.4 / 7.2); up to 16 rows, to 2048 (1280 x 2048 at 16 rows 5.5 / 4.5).  A
 // longer K on fewer than 128 panels, which the panel kernel splits over
 // workgroups that meet through memory, only up to 8 rows (1280 x 5120 at 8 /
-// 16 rows 6.11 / 4.83, 6.5 / 6.9) and, where its four splits are one round of
+// 16 rows 6.11 / 4.83, 6.5 / 6.9; with weights from HBM, not the Infinity Cache
+// that holds a decoder's, 6.5 / 6.9 at 8, 6.2 / 6.1 for 1024 x 4096) and, where its four splits are one round of
 // workgroups (2048 rows of weight), up to 5120 (2048 x 5120 at 8 rows 6.7 /
 // 5.4, x 6144 7.1 / 7.5, 1280 x 12288 9.4 / 12.7, 2176 x 12288 15.8 / 13.4).
 bool skinny16_suits(uint32_t m, uint32_t n, uint32_t k) {
