@@ -606,7 +606,9 @@ void launch_rows(const GemvArgs &a) {
 // Rows per workgroup: 8 while that is at most one workgroup per CU or so,
 // else 16, which halve the x staged per weight (issued from C, us, 8 / 16 /
 // 32 rows: 1280 x 1280 2.5 / 2.7 / -, 3840 x 1280 4.1 / 2.7 / 3.1, 5120 x
-// 1280 5.5 / 3.0 / 3.3, 1280 x 5120 3.6 / 4.5 / -).  One pair of chunks per
+// 1280 5.5 / 3.0 / 3.3, 1280 x 5120 3.6 / 4.5 / -).  The line is that of K =
+// 1280: past K = 4096, where a workgroup holds its CU, 16 rows lead from 2049
+// on (2304 x 5120 with 8 7.2, 2305 x 5120 with 16 5.7).  One pair of chunks per
 // wave up to K = 2048; three, all in flight at once, above (1280 x 1280 with
 // two or three per wave 2.8); past 6144 sixteen waves go round.
 constexpr uint32_t kRows8 = 2304;
